@@ -59,6 +59,23 @@ struct TileQueue {
         return i < queue_lo(ntiles, r + 1) ? i : -1;
     }
 
+    // grab() in two steps, so that the counter's answer can be awaited later:
+    // ask() sends for the next tile of the current range, answer() makes a
+    // tile number of what came back.
+    __device__ int ask(int* q)
+    {
+        return left > 0 ? __hip_atomic_fetch_add(q + r * QSTRIDE, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    }
+    __device__ int answer(int* q, int ntiles, int raw)
+    {
+        if (left <= 0) return ntiles;
+        const int i = queue_lo(ntiles, r) + raw;
+        if (i < queue_lo(ntiles, r + 1)) return i;
+        --left;
+        r = r + 1 == QN ? 0 : r + 1;
+        return grab(q, ntiles);
+    }
+
     // The next tile, or ntiles when every range is empty.
     __device__ int grab(int* q, int ntiles)
     {

@@ -32,6 +32,8 @@ int    batch_family();
 // Batched kernel of family fam and tile-shape index thi (0 .. NBTH-1) for a
 // type pair.
 const BatchEntry& batch_entry(int fam, int thi, int in_dt, int out_dt);
+// Tile-shape index of a batch that has no tuned one.
+int    batch_default(int fam, int in_dt, int out_dt);
 int    make_tiles(std::vector<SepArgs>& jobs, const BatchEntry& e, std::vector<BatchTile>& tiles);
 int    batch_grid(const BatchEntry& e, int ntiles);
 

@@ -142,35 +142,68 @@ icia_mfma_kernel(const SepArgs a, int ntiles, double* __restrict__ partial)
     float* const stage = reinterpret_cast<float*>(stage4) + (threadIdx.x >> 6) * 16 * MOPITCH;
     const int grid = int(gridDim.x);
     int t = xcd_remap(int(blockIdx.x), grid);
-    int y0, x0;
-    bool live = mfma_strip_pos<WY>(a, t, y0, x0);
-    MfmaRaw<IN> raw;
-    if (live) mfma_load<RC, IN>(a, y0, x0, raw);    // in flight while the tables are built
-    mfma_get_tabs<MODE_GAUSS>(a, T);
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < NM; ++k) mom[k * MS] = 0.f;
+    TilePos pos = mfma_tile_pos<WY>(a, t);
     // Radius class 16 takes the lane index afresh in each tile, as the
     // six-output tile loop does (3840 x 2160 u8 projective 3.6 %, 1080p f32
     // affine 2 % faster; radius class 8 within +-1.5 %, so it does not).
     constexpr bool FRESH = RC == 16;
-    while (t < ntiles) {                            // uniform over the workgroup
-        if (live) {
-            v4f32 gH[MNB], gV[MNB];
-            mfma_compute<RC, IN, float, MODE_ICIA, CPOL_NT, FRESH>(
-                a, y0, x0, raw, T, stage, [] {},
-                [&](int k, const v4f32* acc, float u) {
+    const auto strip = [&](const TilePos& at, const MfmaOps& p) {
+        v4f32 gH[MNB], gV[MNB];
+        mfma_filter<RC, IN, float, MODE_ICIA, CPOL_NT, FRESH>(
+            a, at.y0, at.x0, p, T, stage,
+            [&](int k, const v4f32* acc, float u) {
 #pragma unroll
-                    for (int o = 0; o < MNB; ++o) {
-                        if (k == 1) gH[o] = acc[o] * u;
-                        else        gV[o] = acc[o] * u;
-                    }
-                }, a.mask);
-            icia_lane_moments<D>(a, y0, x0, gH, gV, mom, MS);
+                for (int o = 0; o < MNB; ++o) {
+                    if (k == 1) gH[o] = acc[o] * u;
+                    else        gV[o] = acc[o] * u;
+                }
+            }, a.mask, [] {});
+        icia_lane_moments<D>(a, at.y0, at.x0, gH, gV, mom, MS);
+    };
+    if constexpr (sizeof(IN) < 4) {
+        // as the single-image tile loop
+        using W = MWin<RC, WY, MWAVES / WY, IN>;
+        __shared__ v4u32 win4[W::BYTES / 16];
+        char* const win = reinterpret_cast<char*>(win4);
+        v4u32 v[W::N];
+        const int tid = int(threadIdx.x);
+        mwin_load<RC, WY, MWAVES / WY, IN>(a, tid, pos.ty, pos.tx, v);    // in flight while the tables are copied
+        mfma_get_tabs<MODE_GAUSS>(a, T);
+#pragma unroll
+        for (int k = 0; k < NM; ++k) mom[k * MS] = 0.f;
+        for (;;) {                                  // t is uniform over the workgroup
+            mwin_store<RC, WY, MWAVES / WY, IN>(tid, win, v);
+            lds_barrier();                          // the window (at first also the tables) is complete
+            MfmaOps p;
+            if (pos.live) mfma_ops_tile<RC, WY, MWAVES / WY, IN, FRESH>(a, win, p);
+            lds_barrier();                          // every wave has its operands
+            const TilePos now = pos;
+            t += grid;
+            if (t < ntiles) {
+                pos = mfma_tile_pos<WY>(a, t);
+                mwin_load<RC, WY, MWAVES / WY, IN>(a, tid, pos.ty, pos.tx, v);
+            }
+            if (now.live) strip(now, p);
+            if (t >= ntiles) break;
         }
-        t += grid;
-        live = t < ntiles && mfma_strip_pos<WY>(a, t, y0, x0);
-        if (live) mfma_load<RC, IN, FRESH>(a, y0, x0, raw);
+    } else {
+        MfmaRaw raw;
+        if (pos.live) mfma_load<RC>(a, pos.y0, pos.x0, raw);    // in flight while the tables are built
+        mfma_get_tabs<MODE_GAUSS>(a, T);
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < NM; ++k) mom[k * MS] = 0.f;
+        while (t < ntiles) {                        // uniform over the workgroup
+            if (pos.live) {
+                MfmaOps p;
+                mfma_ops_raw<RC>(a, raw, p);
+                strip(pos, p);
+            }
+            t += grid;
+            if (t >= ntiles) break;
+            pos = mfma_tile_pos<WY>(a, t);
+            if (pos.live) mfma_load<RC, FRESH>(a, pos.y0, pos.x0, raw);
+        }
     }
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
 #pragma unroll

@@ -215,125 +215,109 @@ template <int CTRL> __device__ __forceinline__ float dpp_f32(float v)
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
 
-// Largest v over the wave (every lane active), in every lane: DPP within
-// each row of 16 lanes (quad swaps, half-row and row mirrors), then the four
-// row results read as scalars.  (Six ds_bpermute rounds, each waiting for
-// the LDS, did the same with a longer dependent chain.)
+// Largest v over the wave (every lane active), in every lane, NaN if a lane
+// holds one: DPP within each row of 16 lanes (quad swaps, half-row and row
+// mirrors), then the four row results read as scalars.  (Six ds_bpermute
+// rounds, each waiting for the LDS, did the same with a longer dependent
+// chain.)
 __device__ __forceinline__ float wave_max(float v)
 {
-    v = fmaxf(v, dpp_f32<0xb1>(v));             // quad_perm [1, 0, 3, 2]
-    v = fmaxf(v, dpp_f32<0x4e>(v));             // quad_perm [2, 3, 0, 1]
-    v = fmaxf(v, dpp_f32<0x141>(v));            // row_half_mirror
-    v = fmaxf(v, dpp_f32<0x140>(v));            // row_mirror
+    const auto mx = [](float a, float b) { return __builtin_elementwise_maximum(a, b); };
+    v = mx(v, dpp_f32<0xb1>(v));                // quad_perm [1, 0, 3, 2]
+    v = mx(v, dpp_f32<0x4e>(v));                // quad_perm [2, 3, 0, 1]
+    v = mx(v, dpp_f32<0x141>(v));               // row_half_mirror
+    v = mx(v, dpp_f32<0x140>(v));               // row_mirror
     const float a = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 0));
     const float b = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 16));
     const float c = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 32));
     const float d = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 48));
-    return fmaxf(fmaxf(a, b), fmaxf(c, d));
+    return mx(mx(a, b), mx(c, d));
 }
 
-// Two u8 values as f16 times s, exactly: with M = 1024 s a power of two in
-// f16's normal range, M's bits with x (< 256) in the low mantissa bits are
-// the f16 M + x s, and subtracting M leaves x s.  mb = M's bits in both
-// halves, nm = -M in both halves.
-__device__ __forceinline__ v2f16 u8pair_f16(uint32_t lo, uint32_t hi, uint32_t mb, v2f16 nm)
+// A wave's output staging area: 16 rows of 64 pixels in the output's type,
+// the row pitch a multiple of 16 bytes that spreads the rows over the banks;
+// a store instruction takes 16 bytes a lane, RPI rows.
+template <class OUT> struct MStage {
+    static constexpr int ES    = int(sizeof(OUT));
+    static constexpr int PITCH = MSTRIP_W * ES + 16;
+    static constexpr int EPL   = 16 / ES;                   // pixels per lane
+    static constexpr int LPR   = MSTRIP_W / EPL;            // lanes per row
+    static constexpr int RPI   = 64 / LPR;
+    static constexpr int NI    = 16 / RPI;                  // store instructions per output
+    static_assert(PITCH <= MOPITCH * 4, "staging area too narrow");
+};
+
+typedef v4u32 v4u32u __attribute__((aligned(1)));
+
+// Stores the elements [xa, xb) (of 16 / ES, ES bytes each) of q at p.
+template <int ES> __device__ __forceinline__ void store_chunk(uintptr_t p, v4u32 q, int xa, int xb)
 {
-    const uint32_t w = (hi << 16) | lo | mb;
-    return __builtin_bit_cast(v2f16, w) + nm;
+    constexpr int E = 16 / ES;
+    using T = std::conditional_t<ES == 4, uint32_t, std::conditional_t<ES == 2, uint16_t, uint8_t>>;
+    if (xa <= 0 && xb >= E) {
+        *reinterpret_cast<gptr<v4u32u>>(p) = q;
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+        if (e >= xa && e < xb) reinterpret_cast<gptr<T>>(p)[e] = T(q[e * ES / 4] >> (8 * (e * ES % 4)));
 }
 
-// One input value as loaded, unconverted: float, the 16 bits of an f16 /
-// bf16, or the byte.  mfma_compute converts them where it uses them, so that
-// no conversion sits right after the loads and makes the wave wait for them
-// there (the loads of a strip stay in flight through the table build, or
-// through the previous strip's work in the tile loop).
-// Narrow inputs are held zero-extended in 32 bits.
-template <class IN> using RawElem = std::conditional_t<sizeof(IN) == 4, float, uint32_t>;
-
-// Range-checked load of a float input (a pixel outside the image reads 0).
-template <class IN>
-__device__ __forceinline__ RawElem<IN> mfma_ld(__amdgpu_buffer_rsrc_t r, int voff, int soff)
+// Stores S elements (of ES bytes) from LDS through a buffer, at offset at
+// (past the buffer: nothing).
+template <int ES, int S, int CPOL>
+__device__ __forceinline__ void store_piece(__amdgpu_buffer_rsrc_t r, const char* p, int at)
 {
-    static_assert(sizeof(IN) == 4, "narrow inputs load with mfma_ld_in");
-    return Px<IN>::ld(r, voff, soff);
-}
-
-// Unchecked load at row base + lane offset, for windows inside the image:
-// a narrow value arrives zero-extended by the load itself (with the buffer
-// form the compiler masks it again, and that mask, placed right after the
-// loads, makes the wave wait for them there).
-template <class IN>
-__device__ __forceinline__ RawElem<IN> mfma_ld_in(const char* row, uint32_t off)
-{
-    const gptr<const uint8_t> base = reinterpret_cast<gptr<const uint8_t>>(reinterpret_cast<uintptr_t>(row));
-    if constexpr (sizeof(IN) == 4)
-        return *reinterpret_cast<const gptr<const float>>(base + off);
-    else if constexpr (sizeof(IN) == 2)
-        return *reinterpret_cast<const gptr<const uint16_t>>(base + off);
+    if constexpr (S * ES == 8)
+        __builtin_amdgcn_raw_buffer_store_b64(*reinterpret_cast<const v2u32*>(p), r, at, 0, CPOL);
+    else if constexpr (S * ES == 4)
+        __builtin_amdgcn_raw_buffer_store_b32(*reinterpret_cast<const uint32_t*>(p), r, at, 0, CPOL);
+    else if constexpr (S * ES == 2)
+        __builtin_amdgcn_raw_buffer_store_b16(*reinterpret_cast<const uint16_t*>(p), r, at, 0, CPOL);
     else
-        return base[off];
+        __builtin_amdgcn_raw_buffer_store_b8(*reinterpret_cast<const uint8_t*>(p), r, at, 0, CPOL);
 }
 
-// The value of a loaded element as a float.
-template <class IN>
-__device__ __forceinline__ float raw_value(RawElem<IN> v)
-{
-    if constexpr (std::is_same_v<IN, f16_t>)
-        return float(__builtin_bit_cast(_Float16, uint16_t(v)));
-    else if constexpr (std::is_same_v<IN, bf16_t>)
-        return __uint_as_float(uint32_t(v) << 16);
-    else
-        return float(v);
-}
-
-// Input values of field block b for lane (g, m): column x0 - RC + 16 b + m,
-// rows y0 - RC + 8 g + j (j < 8) and, for K = 48, y0 - RC + 32 + 4 g + j
-// (j < 4).  INSIDE: every pixel of the strip's window lies in the image
-// (row offsets as scalar offsets); otherwise pixels outside the image read
-// as 0 (buffer range check for float input; for narrow input a load at the
-// clamped address and a select).
-template <int RC, bool INSIDE, class IN, class A>
+// The elements left of a chunk that an edge cuts, NI row steps of it (rpitch
+// bytes apart in LDS, opitch in the output): its last n (tail) or first n
+// elements, as pieces of E / 2, E / 4, .. 1 elements, each at most once and at
+// a multiple of its size (the bits of n).  at is the chunk's offset; row step
+// i is stored if bit i of rows is set.
+template <int ES, int CPOL, int NI, int S = 8 / ES>
 __device__ __forceinline__ void
-mfma_load_block(const A& a, __amdgpu_buffer_rsrc_t rsrc, int y0, int x0, int b, int g, int m, RawElem<IN>* v)
+store_cut(__amdgpu_buffer_rsrc_t r, const char* src, int rpitch, int at, int opitch, bool tail, int n, unsigned rows)
+{
+    constexpr int E = 16 / ES;
+    const int pos = n & S ? (tail ? E - (n & ~(S - 1)) : n & ~(2 * S - 1)) : 0;
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+        store_piece<ES, S, CPOL>(r, src + pos * ES + i * rpitch,
+                                 (n & S) && (rows >> i & 1u) ? at + pos * ES + i * opitch : MINVALID);
+    if constexpr (S > 1) store_cut<ES, CPOL, NI, S / 2>(r, src, rpitch, at, opitch, tail, n, rows);
+}
+
+// Input values of field block b for lane (g, m), float input: column x0 - RC +
+// 16 b + m, rows y0 - RC + 8 g + j (j < 8) and, for K = 48, y0 - RC + 32 +
+// 4 g + j (j < 4).  INSIDE: every pixel of the strip's window lies in the
+// image (row offsets as scalar offsets); otherwise pixels outside the image
+// read as 0 by the buffer's range check.
+template <int RC, bool INSIDE, class A>
+__device__ __forceinline__ void
+mfma_load_block(const A& a, __amdgpu_buffer_rsrc_t rsrc, int y0, int x0, int b, int g, int m, float* v)
 {
     constexpr int NLD = MGeo<RC>::NLD;
-    const int es = int(sizeof(IN));
+    constexpr int es = int(sizeof(float));
     const int col = x0 - RC + 16 * b + m;
     const int sb = a.in_stride_b;
     const int r0 = y0 - RC + 8 * g;            // first row of entries 0 .. 7
     const int r1 = y0 - RC + 32 + 4 * g;       // first row of entries 8 .. 11
-    if constexpr (INSIDE && sizeof(IN) < 4) {
-        // row bases uniform (y0 - RC + j), lane offsets 32-bit
-        const char* const in = static_cast<const char*>(a.in);
-        const uint32_t o0 = uint32_t(8 * g * sb + col * es), o1 = uint32_t((32 + 4 * g) * sb + col * es);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = mfma_ld_in<IN>(in + int64_t(y0 - RC + j) * sb, o0);
-        if constexpr (MGeo<RC>::K48) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) v[8 + j] = mfma_ld_in<IN>(in + int64_t(y0 - RC + j) * sb, o1);
-        }
-    } else if constexpr (INSIDE) {
+    if constexpr (INSIDE) {
         const int v0 = r0 * sb + col * es, v1 = r1 * sb + col * es;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = mfma_ld<IN>(rsrc, v0, j * sb);
+        for (int j = 0; j < 8; ++j) v[j] = Px<float>::ld(rsrc, v0, j * sb);
         if constexpr (MGeo<RC>::K48) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) v[8 + j] = mfma_ld<IN>(rsrc, v1, j * sb);
-        }
-    } else if constexpr (sizeof(IN) < 4) {
-        // the same extending loads at addresses clamped into the image, and
-        // 0 where the pixel lies outside (so that the values of both paths
-        // meet without a mask after them)
-        const char* const in = static_cast<const char*>(a.in);
-        const bool colok = unsigned(col) < unsigned(a.ncol);
-        const int colc = min(max(col, 0), a.ncol - 1);
-#pragma unroll
-        for (int j = 0; j < NLD; ++j) {
-            const int row = j < 8 ? r0 + j : r1 + (j - 8);
-            const bool ok = colok && unsigned(row) < unsigned(a.nrow);
-            const int rowc = min(max(row, 0), a.nrow - 1);
-            const RawElem<IN> x = mfma_ld_in<IN>(in + int64_t(rowc) * sb, uint32_t(colc * es));
-            v[j] = ok ? x : 0u;
+            for (int j = 0; j < 4; ++j) v[8 + j] = Px<float>::ld(rsrc, v1, j * sb);
         }
     } else {
         const bool colok = unsigned(col) < unsigned(a.ncol);
@@ -341,10 +325,140 @@ mfma_load_block(const A& a, __amdgpu_buffer_rsrc_t rsrc, int y0, int x0, int b, 
         for (int j = 0; j < NLD; ++j) {
             const int row = j < 8 ? r0 + j : r1 + (j - 8);
             const bool ok = colok && unsigned(row) < unsigned(a.nrow);
-            v[j] = mfma_ld<IN>(rsrc, ok ? row * sb + col * es : MINVALID, 0);
+            v[j] = Px<float>::ld(rsrc, ok ? row * sb + col * es : MINVALID, 0);
         }
     }
 }
+
+// ------------------------------------------------------------ input window
+// u8, f16 and bf16 input reaches the strips through LDS: the workgroup loads
+// the window of its tile (SY strips down by SX across, and the radius class
+// around them) once, as stored, with 16-byte loads, and each strip reads its
+// matrix operands from there with the transposing LDS reads (ds_read_b64_tr:
+// within 16 lanes, lane i supplies the address of 8 bytes and receives column
+// i of the 4 rows of 16-bit or 8 rows of 8-bit elements they cover), which
+// hand each lane the 8 rows of one column that a vertical product takes as
+// its K entries.  One load per pixel and lane (40 or 72 per strip, each
+// touching four rows for 64 or 128 bytes) kept the address units busy for a
+// fifth of a launch, held 40 - 72 registers, and read the rows that
+// neighbouring strips share once per strip.
+// Pixels outside the image are 0 in the window.
+template <int RC, int SY, int SX, class IN>
+struct MWin {
+    static constexpr int ES    = int(sizeof(IN));
+    static constexpr int ROWS  = 16 * SY + 2 * RC;
+    static constexpr int COLS  = 16 * (MNB * SX + MGeo<RC>::NVB - MNB);
+    static constexpr int PITCH = COLS * ES;                 // bytes, a multiple of 16
+    static constexpr int CPR   = PITCH / 16;                // 16-byte chunks per row
+    static constexpr int NC    = ROWS * CPR;
+    static constexpr int NT_   = 64 * SY * SX;              // threads of the workgroup
+    static constexpr int N     = (NC + NT_ - 1) / NT_;      // chunks per thread
+    static constexpr int EPC   = 16 / ES;                   // elements per chunk
+    // u8 at radius class 16: the 8-row transposing reads of the last 16 rows
+    // take 4 rows more than they use
+    static constexpr int BYTES = PITCH * (ROWS + (ES == 1 && MGeo<RC>::K48 ? 4 : 0));
+};
+
+// v shifted by d elements of ES bytes: result element j = element j + d of v,
+// 0 where that lies outside.
+template <int ES> __device__ __forceinline__ v4u32 shift_chunk(v4u32 v, int d)
+{
+    uint64_t lo = uint64_t(v[1]) << 32 | v[0], hi = uint64_t(v[3]) << 32 | v[2];
+    const int r = max(d, 0) * (8 * ES), l = max(-d, 0) * (8 * ES);   // at most one is nonzero
+    // right, then left, by 64 and by the rest (x << 1 << (63 - k) is x <<
+    // (64 - k), and 0 for k = 0)
+    const int r1 = r & 63, l1 = l & 63;
+    const uint64_t a0 = r >= 64 ? hi : lo, a1 = r >= 64 ? 0 : hi;
+    lo = a0 >> r1 | a1 << 1 << (63 - r1);
+    hi = a1 >> r1;
+    const uint64_t b1 = l >= 64 ? lo : hi, b0 = l >= 64 ? 0 : lo;
+    hi = b1 << l1 | b0 >> 1 >> (63 - l1);
+    lo = b0 << l1;
+    const bool in = r < 128 && l < 128;
+    return in ? v4u32{uint32_t(lo), uint32_t(lo >> 32), uint32_t(hi), uint32_t(hi >> 32)} : v4u32{0, 0, 0, 0};
+}
+
+// Issues the loads of the window whose tile's first strip is at (y0, x0);
+// every thread (tid) of the workgroup calls it, the chunks arrive in v.
+template <int RC, int SY, int SX, class IN, class A>
+__device__ __forceinline__ void mwin_load(const A& a, int tid, int y0, int x0, v4u32* v)
+{
+    using W = MWin<RC, SY, SX, IN>;
+    const int yw = y0 - RC, xw = x0 - RC, sb = a.in_stride_b;
+    const char* const in = static_cast<const char*>(a.in);
+    const bool inside = yw >= 0 && yw + W::ROWS <= a.nrow && xw >= 0 && xw + W::COLS <= a.ncol;   // uniform
+    if (inside) {
+        const char* const base = in + int64_t(yw) * sb + xw * W::ES;
+#pragma unroll
+        for (int i = 0; i < W::N; ++i) {
+            const int c = min(tid + i * W::NT_, W::NC - 1);
+            const int r = c / W::CPR, q = c - r * W::CPR;
+            v[i] = *reinterpret_cast<gptr<const v4u32u>>(reinterpret_cast<uintptr_t>(base + uint32_t(r * sb + 16 * q)));
+        }
+        return;
+    }
+    // Rows and chunks clamped into the image, then moved to their place: a
+    // chunk that straddles an edge keeps the pixels inside.
+    const bool narrow = a.ncol < W::EPC;                    // uniform: no whole chunk in a row
+    const auto at = [&](int i, int& row, int& col, int& cc) {
+        const int c = min(tid + i * W::NT_, W::NC - 1);
+        const int r = c / W::CPR, q = c - r * W::CPR;
+        row = yw + r;
+        col = xw + W::EPC * q;
+        cc = min(max(col, 0), max(a.ncol - W::EPC, 0));
+        return reinterpret_cast<uintptr_t>(in + int64_t(min(max(row, 0), a.nrow - 1)) * sb);
+    };
+    int row, col, cc;
+    if (!narrow) {
+#pragma unroll
+        for (int i = 0; i < W::N; ++i) {
+            const uintptr_t line = at(i, row, col, cc);
+            v[i] = *reinterpret_cast<gptr<const v4u32u>>(line + uintptr_t(cc * W::ES));
+        }
+    } else {                                                // byte by byte
+#pragma unroll
+        for (int i = 0; i < W::N; ++i) {
+            const gptr<const uint8_t> p = reinterpret_cast<gptr<const uint8_t>>(at(i, row, col, cc));
+            uint64_t lo = 0, hi = 0;
+#pragma unroll 1
+            for (int j = 0; j < a.ncol * W::ES; ++j) {
+                const uint64_t x = uint64_t(p[j]) << (8 * (j & 7));
+                lo |= j < 8 ? x : 0;
+                hi |= j < 8 ? 0 : x;
+            }
+            v[i] = v4u32{uint32_t(lo), uint32_t(lo >> 32), uint32_t(hi), uint32_t(hi >> 32)};
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < W::N; ++i) {
+        (void)at(i, row, col, cc);
+        const v4u32 x = shift_chunk<W::ES>(v[i], col - cc);
+        v[i] = unsigned(row) < unsigned(a.nrow) ? x : v4u32{0, 0, 0, 0};
+    }
+}
+
+// Writes the loaded chunks into the workgroup's window in LDS.
+template <int RC, int SY, int SX, class IN>
+__device__ __forceinline__ void mwin_store(int tid, char* win, const v4u32* v)
+{
+    using W = MWin<RC, SY, SX, IN>;
+#pragma unroll
+    for (int i = 0; i < W::N; ++i)
+        *reinterpret_cast<v4u32*>(win + 16 * min(tid + i * W::NT_, W::NC - 1)) = v[i];
+}
+
+// A barrier that orders the workgroup's LDS accesses only: loads from and
+// stores to memory stay in flight across it.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <class T> using lptr = T __attribute__((address_space(3)))*;   // LDS
+typedef short v4i16 __attribute__((ext_vector_type(4)));
+typedef int v2i32 __attribute__((ext_vector_type(2)));
 
 // f16 hi / lo split of 4 floats times s.
 __device__ __forceinline__ void split4(float v0, float v1, float v2, float v3, float s, v4f16& hi, v4f16& lo)
@@ -418,9 +532,9 @@ __device__ __forceinline__ float fp32_taps(const C& t, int r, const W& w)
 // c_l(k) at 17 l + k; MODE_TAPS the full vertical taps at 16 + o and the
 // horizontal ones at 33 + 16 + o, which for FIRFilter2 lobes (sgnv, sgnh
 // nonzero) are c(k) on the upper / left side.
-template <int RC, class IN, class OUT, int MODE, class A>
+template <int RC, class IN, class OUT, int MODE>
 __device__ __forceinline__ void
-mfma_strip_fp32(const A& a, int y0, int x0, const MfmaTabs& T, float* stage, unsigned mask)
+mfma_strip_fp32(ConstArgs& a, int y0, int x0, const MfmaTabs& T, float* stage, unsigned mask)
 {
     constexpr bool ONE = MODE == MODE_TAPS;
     constexpr int NFC = 32 + 2 * RC;            // field columns per half strip
@@ -429,6 +543,9 @@ mfma_strip_fp32(const A& a, int y0, int x0, const MfmaTabs& T, float* stage, uns
     // path is computed ahead of it (in a tile loop, such hoisted values would
     // hold registers across the matrix-core path).
     int lane = threadIdx.x & 63;
+    y0 = __builtin_amdgcn_readfirstlane(y0);
+    x0 = __builtin_amdgcn_readfirstlane(x0);
+    mask = __builtin_amdgcn_readfirstlane(mask);
     asm volatile("" : "+v"(lane), "+s"(y0), "+s"(x0), "+s"(mask));
     const int es = int(sizeof(IN));
     const int sb = a.in_stride_b;
@@ -500,50 +617,63 @@ mfma_strip_fp32(const A& a, int y0, int x0, const MfmaTabs& T, float* stage, uns
     }
 }
 
+// The arguments behind a pointer the compiler cannot see through, so that it
+// reads those of the rarely taken FP32 form there, and not before the strip
+// code, where they would hold 40 scalar registers: a job's in device memory,
+// or the kernel's own (every matrix-core kernel's first argument).
+__device__ __forceinline__ ConstArgs& opaque_args(ConstArgs& a)
+{
+    const uintptr_t p = (uintptr_t)&a;
+    uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(p)), hi = __builtin_amdgcn_readfirstlane(uint32_t(p >> 32));
+    asm volatile("" : "+s"(lo), "+s"(hi));
+    return *(ConstArgs*)(uintptr_t(hi) << 32 | lo);
+}
+__device__ __forceinline__ ConstArgs& opaque_args(const SepArgs&)
+{
+    uintptr_t p = (uintptr_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(ConstArgs*)p;
+}
+
 #define TUCU_MFMA(A_, B_, C_) __builtin_amdgcn_mfma_f32_16x16x32_f16((A_), (B_), (C_), 0, 0, 0)
 
-// One strip: centre rows y0 .. y0+15, centre columns x0 .. x0+63.  T holds
-// the operand runs (mfma_build_tabs).  Every lane of the wave calls it.
-//
-// Operand layouts (lane = 16 g + m; m is also the row / output column n):
-//   vertical, block b, K32 slice: A = input rows y0 - RC + 8 g + j (j < 8)
-//     of column x0 - RC + 16 b + m; B = taps of offsets 8 g + j - RC - n.
-//   vertical, K48 second slice: A = rows 32 + 4 g .. +3 of the lane's
-//     input, high halves then low halves; B = taps of offsets
-//     32 + 4 g + j - RC - n twice (high taps: both halves of the input in
-//     one product), or once and then zeros (low taps x high input).
-//   horizontal, K32 (radius class 8), output block o: B = field blocks o,
-//     o + 1 (lane holds columns 4 g .. 4 g + 3 of each, window columns
-//     4 g + j and 16 + 4 g + j); A = taps of offsets (window column) - RC - m.
-//   horizontal, K48: two K32 slices over the fixed pairs P_(o/2) and
-//     P_(o/2 + 1) of field blocks (2 p, 2 p + 1); A = taps as above, shifted
-//     by d = 32 p - 16 o (zero for the block outside the window).
-// A strip's input, as loaded: field block b, entry j (mfma_load_block's
-// order); radius class 8 uses blocks 0 .. 4 and entries 0 .. 7.
-template <class IN> using MfmaRaw = RawElem<IN>[6][12];
+// A strip's float input, as loaded: field block b, entry j
+// (mfma_load_block's order); radius class 8 uses blocks 0 .. 4 and entries
+// 0 .. 7.
+using MfmaRaw = float[6][12];
 
-// Register budget of the kernels: two waves per SIMD for float input (the
-// low halves of the input and of the tail rows stay live), three for 16-bit
-// and u8 input (exact in one f16; measured 9 % faster in the batched mode).
-// The single-image tile loop keeps two: inlined in a loop the strip code
-// needs more registers.
-template <class IN> constexpr int MFMA_WAVES_PER_SIMD = sizeof(IN) == 4 ? 2 : 3;
+// A strip's matrix operands of the vertical pass, and its scale.
+// xh / xl: entries 0 .. 7 (rows 8 g + j), high and low halves; xt (K = 48):
+// entries 8 .. 11 (rows 32 + 4 g + j), high then low halves, so that one
+// product with the high taps twice covers both halves of those rows.
+// Inputs exact in f16 have no low half: xt then holds the high halves
+// twice, and one product with the high and the low taps side by side
+// covers both tap halves (one product per block instead of two).
+struct MfmaOps {
+    v8f16 xh[6], xl[6], xt[6];  // field blocks; radius class 8 uses 0 .. 4
+    float inv_s;                // undoes the strip's scale
+    bool  redo;                 // the products cannot carry the input: the FP32 form filters the strip
+};
 
-// The single-image tile loop (large images): two waves per SIMD for the
-// six-output Gaussian (the strip code inlined in a loop needs more
-// registers); the one-output mode (FIRFilter2 lobes, general taps) needs
-// fewer, but at three or four waves per SIMD it spills (176-236 bytes per
-// lane at four): two by default, TUCU_LOOP_WAVES_TAPS at build time to try.
-#ifndef TUCU_LOOP_WAVES_TAPS
-#define TUCU_LOOP_WAVES_TAPS 2
-#endif
-template <int MODE, class IN> constexpr int MFMA_LOOP_WAVES = MODE == MODE_TAPS ? TUCU_LOOP_WAVES_TAPS : 2;
+// Register budget of the kernels: three waves per SIMD (the one-round and
+// batched float kernels need 160 - 169 registers; 64 batched 1080p images f32
+// 12.2 us each against 13.0 at two waves).  The single-image tile loop of
+// float input keeps two: inlined in a loop the strip code needs more registers.
+constexpr int MFMA_WAVES_PER_SIMD = 3;
 
-// Issues the loads of the strip at (y0, x0); the values arrive in raw.
+// The single-image tile loop (large images): the float strip code inlined in
+// a loop needs more registers than the one-round kernels, two waves per SIMD
+// (the one-output mode needs fewer, but at three or four it spills);
+// narrow input, which holds no float values and prefetches the next window
+// in at most 20 registers, takes three at radius class 16 (four by itself
+// where it needs 128 registers or fewer).
+template <class IN> constexpr int MFMA_LOOP_WAVES = sizeof(IN) == 4 ? 2 : 3;
+
+// Issues the loads of the float strip at (y0, x0); the values arrive in raw.
 // FRESH: the lane index is opaque to the compiler (a caller's loop then
 // recomputes what derives from it in each pass instead of holding it).
-template <int RC, class IN, bool FRESH = false, class A>
-__device__ __forceinline__ void mfma_load(const A& a, int y0, int x0, MfmaRaw<IN>& raw)
+template <int RC, bool FRESH = false, class A>
+__device__ __forceinline__ void mfma_load(const A& a, int y0, int x0, MfmaRaw& raw)
 {
     using G = MGeo<RC>;
     int lane = threadIdx.x & 63;
@@ -558,10 +688,10 @@ __device__ __forceinline__ void mfma_load(const A& a, int y0, int x0, MfmaRaw<IN
                         x0 - RC >= 0 && x0 - RC + 16 * G::NVB <= a.ncol;
     if (inside) {
 #pragma unroll
-        for (int b = 0; b < G::NVB; ++b) mfma_load_block<RC, true, IN>(a, rsrc, y0, x0, b, g, m, raw[b]);
+        for (int b = 0; b < G::NVB; ++b) mfma_load_block<RC, true>(a, rsrc, y0, x0, b, g, m, raw[b]);
     } else {
 #pragma unroll
-        for (int b = 0; b < G::NVB; ++b) mfma_load_block<RC, false, IN>(a, rsrc, y0, x0, b, g, m, raw[b]);
+        for (int b = 0; b < G::NVB; ++b) mfma_load_block<RC, false>(a, rsrc, y0, x0, b, g, m, raw[b]);
     }
     if constexpr (!G::K48) {
 #pragma unroll
@@ -569,11 +699,175 @@ __device__ __forceinline__ void mfma_load(const A& a, int y0, int x0, MfmaRaw<IN
     }
 }
 
-// One strip: centre rows y0 .. y0+15, centre columns x0 .. x0+63, input in
-// raw (mfma_load).  T holds the operand runs (mfma_build_tabs), stage is the
-// wave's output staging area.  after_vpass() runs once raw has been
-// consumed (it may reuse raw, e.g. to prefetch the next strip).  Every lane
-// of the wave calls it.
+// Power-of-two scale of a strip whose largest magnitude (over the wave) is
+// mx: the exponent ex puts it in [2^12, 2^13).  Strips whose largest magnitude
+// is below 2^-87 or above 2^113 are out of the scale's reach (their scaled
+// values would lose precision or overflow f16), and strips with a NaN or an
+// Inf (mx is then one) would spread it: the FP32 form filters them.
+__device__ __forceinline__ int mfma_scale_exp(float mx, bool& redo)
+{
+    int ex;
+    (void)frexpf(mx, &ex);                      // mx < 2^ex
+    ex = 13 - ex;
+    redo = ex < -100 || ex > 100 || !(mx <= 3.4e38f);
+    return ex;
+}
+
+// The operands of a float strip from its loaded values.
+template <int RC, class A>
+__device__ __forceinline__ void mfma_ops_raw(const A& a, const MfmaRaw& raw, MfmaOps& p)
+{
+    using G = MGeo<RC>;
+    float mx = 0.f;
+#pragma unroll
+    for (int b = 0; b < G::NVB; ++b)
+#pragma unroll
+        for (int j = 0; j < G::NLD; ++j) mx = __builtin_elementwise_maximum(mx, fabsf(raw[b][j]));   // keeps a NaN
+    const int ex = mfma_scale_exp(wave_max(mx), p.redo);
+    const float s = ldexpf(a.mq, ex);
+    p.inv_s = ldexpf(1.f, -ex);
+#pragma unroll
+    for (int b = 0; b < G::NVB; ++b) {
+        v4f16 h0, l0, h1, l1;
+        const float* const r = raw[b];
+        split4(r[0], r[1], r[2], r[3], s, h0, l0);
+        split4(r[4], r[5], r[6], r[7], s, h1, l1);
+        p.xh[b] = cat8(h0, h1);
+        p.xl[b] = cat8(l0, l1);
+        if constexpr (G::K48) {
+            v4f16 h2, l2;
+            split4(r[8], r[9], r[10], r[11], s, h2, l2);
+            p.xt[b] = cat8(h2, l2);
+        }
+    }
+}
+
+// Two 16-bit values as stored times s, in f16 (round to nearest even): the
+// multiplication and the conversion in one mixed-precision FMA each.
+template <class IN> __device__ __forceinline__ v2f16 scale_pair(uint32_t w, float s, float zero)
+{
+    float lo, hi;
+    if constexpr (std::is_same_v<IN, bf16_t>) {
+        lo = __uint_as_float(w << 16);
+        hi = __uint_as_float(w & 0xffff0000u);
+    } else {
+        const v2f16 h = __builtin_bit_cast(v2f16, w);
+        lo = float(h[0]);
+        hi = float(h[1]);
+    }
+    return v2f16{_Float16(__builtin_fmaf(lo, s, zero)), _Float16(__builtin_fmaf(hi, s, zero))};
+}
+
+// Two u8 values (bytes I, I + 1 of w) as f16 times s, exactly: with M = 1024 s
+// a power of two in f16's normal range, M's bits with x (< 256) in the low
+// mantissa bits are the f16 M + x s, and subtracting M leaves x s.  mb = M's
+// bits in both halves (the low byte of each is 0), nm = -M in both halves.
+template <int I> __device__ __forceinline__ v2f16 u8pair_f16(uint32_t w, uint32_t mb, v2f16 nm)
+{
+    // v_perm selector: bytes 0 - 3 of the second source, 4 - 7 of the first
+    constexpr uint32_t sel = uint32_t(I) | 5u << 8 | uint32_t(I + 1) << 16 | 7u << 24;
+    return __builtin_bit_cast(v2f16, __builtin_amdgcn_perm(mb, w, sel)) + nm;
+}
+
+// The operands of a narrow strip from the window in LDS (row pitch PITCH
+// bytes); win is the window's byte at the first row and column of the strip's
+// own window.
+template <int RC, class IN, int PITCH, class A>
+__device__ __forceinline__ void mfma_ops_win(const A& a, const char* win, int lane, MfmaOps& p)
+{
+    using G = MGeo<RC>;
+    constexpr int NVB = G::NVB;
+    const int g = lane >> 4, i = lane & 15;
+    if constexpr (std::is_same_v<IN, uint8_t>) {
+        // The scale of 255 (2^5) whatever the strip holds: every byte times
+        // 2^5 mq is exact in f16, and the error bound, relative to 255, stays
+        // that of the brightest strip.  s lies in [2^-7, 2^5] (mq in
+        // [2^-12, 1]), so M = 1024 s is a normal f16.
+        constexpr int ex = 5;
+        p.redo = false;
+        p.inv_s = ldexpf(1.f, -ex);
+        const _Float16 M = _Float16(1024.f * ldexpf(a.mq, ex));
+        const uint32_t mb = uint32_t(__builtin_bit_cast(uint16_t, M)) * 0x10001u;
+        const v2f16 nm = {-M, -M};
+        const char* const w0 = win + (8 * g + i / 2) * PITCH + 8 * (i % 2);
+        const char* const w1 = win + (32 + 4 * g + i / 2) * PITCH + 8 * (i % 2);
+#pragma unroll
+        for (int b = 0; b < NVB; ++b) {
+            const v2i32 d = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lptr<v2i32>)(w0 + 16 * b));
+            const v2f16 p0 = u8pair_f16<0>(d[0], mb, nm), p1 = u8pair_f16<2>(d[0], mb, nm);
+            const v2f16 p2 = u8pair_f16<0>(d[1], mb, nm), p3 = u8pair_f16<2>(d[1], mb, nm);
+            p.xh[b] = v8f16{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
+            if constexpr (G::K48) {
+                const v2i32 e = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lptr<v2i32>)(w1 + 16 * b));
+                const v2f16 p4 = u8pair_f16<0>(e[0], mb, nm), p5 = u8pair_f16<2>(e[0], mb, nm);
+                p.xt[b] = v8f16{p4[0], p4[1], p5[0], p5[1], p4[0], p4[1], p5[0], p5[1]};
+            }
+        }
+    } else {
+        constexpr int NP = G::NLD / 2;          // pairs of rows per lane and block
+        typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+        uint32_t d[NVB][NP];
+        const char* const w0 = win + (8 * g + i / 4) * PITCH + 8 * (i % 4);
+        const char* const w1 = win + (32 + 4 * g + i / 4) * PITCH + 8 * (i % 4);
+        const auto rd = [](const char* q) {
+            return __builtin_bit_cast(v2u, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lptr<v4i16>)q));
+        };
+#pragma unroll
+        for (int b = 0; b < NVB; ++b) {
+            const v2u x = rd(w0 + 32 * b), y = rd(w0 + 32 * b + 4 * PITCH);
+            d[b][0] = x[0]; d[b][1] = x[1]; d[b][2] = y[0]; d[b][3] = y[1];
+            if constexpr (G::K48) {
+                const v2u z = rd(w1 + 32 * b);
+                d[b][4] = z[0]; d[b][5] = z[1];
+            }
+        }
+        // largest magnitude, a NaN if there is one
+        float mx = 0.f;
+        if constexpr (std::is_same_v<IN, bf16_t>) {
+            // the upper value of a pair with the lower one's bits below its
+            // own: they change neither its exponent nor what is not finite
+#pragma unroll
+            for (int b = 0; b < NVB; ++b)
+#pragma unroll
+                for (int j = 0; j < NP; ++j)
+                    mx = __builtin_elementwise_maximum(
+                        __builtin_elementwise_maximum(mx, fabsf(__uint_as_float(d[b][j] << 16))),
+                        fabsf(__uint_as_float(d[b][j])));
+        } else {
+            v2f16 m2 = {0, 0};
+#pragma unroll
+            for (int b = 0; b < NVB; ++b)
+#pragma unroll
+                for (int j = 0; j < NP; ++j) {
+                    const v2f16 h = __builtin_bit_cast(v2f16, d[b][j]);
+                    m2 = __builtin_elementwise_maximum(__builtin_elementwise_maximum(m2, h), -h);
+                }
+            mx = __builtin_elementwise_maximum(float(m2[0]), float(m2[1]));
+        }
+        const int ex = mfma_scale_exp(wave_max(mx), p.redo);
+        const float s = ldexpf(a.mq, ex);
+        p.inv_s = ldexpf(1.f, -ex);
+        float zero = 0.f;                       // opaque: x s + 0 stays one mixed-precision FMA
+        asm("" : "+v"(zero));
+#pragma unroll
+        for (int b = 0; b < NVB; ++b) {
+            v2f16 h[NP];
+#pragma unroll
+            for (int j = 0; j < NP; ++j) h[j] = scale_pair<IN>(d[b][j], s, zero);
+            p.xh[b] = v8f16{h[0][0], h[0][1], h[1][0], h[1][1], h[2][0], h[2][1], h[3][0], h[3][1]};
+            if constexpr (G::K48)
+                p.xt[b] = v8f16{h[4][0], h[4][1], h[5][0], h[5][1], h[4][0], h[4][1], h[5][0], h[5][1]};
+        }
+    }
+}
+
+// One strip: centre rows y0 .. y0+15, centre columns x0 .. x0+63, its
+// operands in p.  T holds the operand runs (mfma_build_tabs), stage is the
+// wave's output staging area.  Every lane of the wave calls it.
+// before_store() runs once, before the strip's first stores: a tile loop
+// waits there for the next window's loads.  The wait counter of a wave
+// covers loads and stores in order, so after this tile's stores it would
+// wait for them too; there it covers only the previous tile's.
 //
 // Operand layouts (lane = 16 g + m; m is also the row / output column n):
 //   vertical, block b, K32 slice: A = input rows y0 - RC + 8 g + j (j < 8)
@@ -588,15 +882,14 @@ __device__ __forceinline__ void mfma_load(const A& a, int y0, int x0, MfmaRaw<IN
 //   horizontal, K48: two K32 slices over the fixed pairs P_(o/2) and
 //     P_(o/2 + 1) of field blocks (2 p, 2 p + 1); A = taps as above, shifted
 //     by d = 32 p - 16 o (zero for the block outside the window).
-template <int RC, class IN, class OUT, int MODE = MODE_GAUSS, int CPOL = CPOL_NT, bool FRESH = false, class A, class F,
-          class S>
+template <int RC, class IN, class OUT, int MODE = MODE_GAUSS, int CPOL = CPOL_NT, bool FRESH = false, class A, class S, class H>
 __device__ __forceinline__ void
-mfma_compute(const A& a, int y0, int x0, MfmaRaw<IN>& raw, const MfmaTabs& T, float* stage, F&& after_vpass,
-             S&& sink, unsigned mask)
+mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const MfmaTabs& T, float* stage, S&& sink, unsigned mask,
+            H&& before_store)
 {
     constexpr bool ONE = MODE == MODE_TAPS;     // one field (table 0), one output (table 1 across)
     using G = MGeo<RC>;
-    constexpr int NVB = G::NVB, NLD = G::NLD;
+    constexpr int NVB = G::NVB;
     constexpr bool XLO = sizeof(IN) == 4;       // f16 / bf16 / u8 inputs are exact in one f16
     constexpr int NF = 4 * NVB;                 // field entries per lane
     typedef _Float16 vfield __attribute__((ext_vector_type(NF)));
@@ -604,71 +897,8 @@ mfma_compute(const A& a, int y0, int x0, MfmaRaw<IN>& raw, const MfmaTabs& T, fl
     if constexpr (FRESH) asm volatile("" : "+v"(lane));    // as for mfma_load
     const int g = lane >> 4, m = lane & 15;
     const v4f16 z4 = {0, 0, 0, 0};
-
-    constexpr bool U8 = std::is_same_v<IN, uint8_t>;
-    // Scale exponent: the largest scaled input in [2^12, 2^13).  u8 input
-    // takes the one for 255 (2^5) whatever the strip holds: every byte
-    // times 2^5 mq is exact in f16, and the error bound, relative to 255,
-    // stays that of the brightest strip.
-    int ex = 5;
-    if constexpr (!U8) {
-        float mx = 0.f;
-#pragma unroll
-        for (int b = 0; b < NVB; ++b)
-#pragma unroll
-            for (int j = 0; j < NLD; ++j) mx = fmaxf(mx, fabsf(raw_value<IN>(raw[b][j])));
-        mx = wave_max(mx);
-        (void)frexpf(mx, &ex);                  // mx < 2^ex
-        ex = 13 - ex;
-    }
-    // Strips whose largest magnitude is below 2^-87 or above 2^113 are out
-    // of the scale's reach (their scaled values would lose precision or
-    // overflow f16): the FP32 form filters them.  u8 input never is.
-    constexpr bool CHECK = !U8 && MODE != MODE_ICIA;
-    bool redo = CHECK && (ex < -100 || ex > 100);   // wave-uniform
-    const float s = ldexpf(a.mq, ex), inv_s = ldexpf(1.f, -ex);
-
-    // xh / xl: entries 0 .. 7 (rows 8 g + j), high and low halves; xt (K = 48):
-    // entries 8 .. 11 (rows 32 + 4 g + j), high then low halves, so that one
-    // product with the high taps twice covers both halves of those rows.
-    // Inputs exact in f16 have no low half: xt then holds the high halves
-    // twice, and one product with the high and the low taps side by side
-    // covers both tap halves (one product per block instead of two)
-    v8f16 xh[NVB], xl[NVB], xt[NVB];
-    if constexpr (U8) {
-        // s = 2^5 mq lies in [2^-7, 2^5] (mq in [2^-12, 1]), so M = 1024 s
-        // is a normal f16
-        const _Float16 M = _Float16(1024.f * s);
-        const uint32_t mb = uint32_t(__builtin_bit_cast(uint16_t, M)) * 0x10001u;
-        const v2f16 nm = {-M, -M};
-#pragma unroll
-        for (int b = 0; b < NVB; ++b) {
-            const v2f16 p0 = u8pair_f16(raw[b][0], raw[b][1], mb, nm), p1 = u8pair_f16(raw[b][2], raw[b][3], mb, nm);
-            const v2f16 p2 = u8pair_f16(raw[b][4], raw[b][5], mb, nm), p3 = u8pair_f16(raw[b][6], raw[b][7], mb, nm);
-            xh[b] = v8f16{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-            if constexpr (G::K48) {
-                const v2f16 p4 = u8pair_f16(raw[b][8], raw[b][9], mb, nm);
-                const v2f16 p5 = u8pair_f16(raw[b][10], raw[b][11], mb, nm);
-                xt[b] = v8f16{p4[0], p4[1], p5[0], p5[1], p4[0], p4[1], p5[0], p5[1]};
-            }
-        }
-    } else {
-#pragma unroll
-        for (int b = 0; b < NVB; ++b) {
-            v4f16 h0, l0, h1, l1;
-            const auto r = [&](int j) { return raw_value<IN>(raw[b][j]); };
-            split4(r(0), r(1), r(2), r(3), s, h0, l0);
-            split4(r(4), r(5), r(6), r(7), s, h1, l1);
-            xh[b] = cat8(h0, h1);
-            xl[b] = cat8(l0, l1);
-            if constexpr (G::K48) {
-                v4f16 h2, l2;
-                split4(r(8), r(9), r(10), r(11), s, h2, l2);
-                xt[b] = cat8(h2, XLO ? l2 : h2);        // 16-bit inputs: lo is 0
-            }
-        }
-    }
-    after_vpass();
+    constexpr bool CHECK = !std::is_same_v<IN, uint8_t> && MODE != MODE_ICIA;   // u8 input is always in range
+    const float inv_s = p.inv_s;
 
     // --------------------------------------------------- vertical pass
     // fh[l] / fl[l]: entries 4 b .. 4 b + 3 = field l at row y0 + n, columns
@@ -679,10 +909,7 @@ mfma_compute(const A& a, int y0, int x0, MfmaRaw<IN>& raw, const MfmaTabs& T, fl
     // and another convert)
     float one = 1.f;
     asm("" : "+v"(one));
-    // vpass(l, ...) also returns, when `sum` is set, the sum of the field's
-    // values: a NaN or an Inf among the strip's inputs makes it non-finite
-    // (every input of a block meets every band entry in the products).
-    auto vpass = [&](int l, vfield& fh, vfield& fl, bool sum) {
+    auto vpass = [&](int l, vfield& fh, vfield& fl) {
         const int t1 = MBASE + 8 * g - RC - m;
         const v8f16 ch1 = cat8(T.run[(0 * 3 + l) * MT4 + t1], T.run[(0 * 3 + l) * MT4 + t1 + 4]);
         const v8f16 cl1 = cat8(T.run[(1 * 3 + l) * MT4 + t1], T.run[(1 * 3 + l) * MT4 + t1 + 4]);
@@ -700,46 +927,55 @@ mfma_compute(const A& a, int y0, int x0, MfmaRaw<IN>& raw, const MfmaTabs& T, fl
         // smaller products first
         if constexpr (XLO) {
 #pragma unroll
-            for (int b = 0; b < NVB; ++b) acc[b] = TUCU_MFMA(xl[b], ch1, acc[b]);
+            for (int b = 0; b < NVB; ++b) acc[b] = TUCU_MFMA(p.xl[b], ch1, acc[b]);
         }
 #pragma unroll
-        for (int b = 0; b < NVB; ++b) acc[b] = TUCU_MFMA(xh[b], cl1, acc[b]);
+        for (int b = 0; b < NVB; ++b) acc[b] = TUCU_MFMA(p.xh[b], cl1, acc[b]);
         if constexpr (G::K48) {
             if constexpr (XLO) {
 #pragma unroll
-                for (int b = 0; b < NVB; ++b) acc[b] = TUCU_MFMA(xt[b], clt, acc[b]);   // hi x lo taps
+                for (int b = 0; b < NVB; ++b) acc[b] = TUCU_MFMA(p.xt[b], clt, acc[b]);   // hi x lo taps
             }
             // XLO: (hi + lo) x hi taps; otherwise hi x (hi + lo taps)
 #pragma unroll
-            for (int b = 0; b < NVB; ++b) acc[b] = TUCU_MFMA(xt[b], cht, acc[b]);
+            for (int b = 0; b < NVB; ++b) acc[b] = TUCU_MFMA(p.xt[b], cht, acc[b]);
         }
 #pragma unroll
-        for (int b = 0; b < NVB; ++b) acc[b] = TUCU_MFMA(xh[b], ch1, acc[b]);
-        float total = 0.f;
-        if (sum) {
-#pragma unroll
-            for (int b = 0; b < NVB; ++b) total += (acc[b][0] + acc[b][1]) + (acc[b][2] + acc[b][3]);
-        }
+        for (int b = 0; b < NVB; ++b) acc[b] = TUCU_MFMA(p.xh[b], ch1, acc[b]);
 #pragma unroll
         for (int b = 0; b < NVB; ++b) {
-            v4f16 h, lo;
-            // hi = f16(v), lo = f16(v - hi): one mixed-precision fma each
-            h = __builtin_convertvector(acc[b], v4f16);
+            const v4f16 h = __builtin_convertvector(acc[b], v4f16);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) lo[i] = _Float16(__builtin_fmaf(acc[b][i], one, -float(h[i])));
-#pragma unroll
-            for (int i = 0; i < 4; ++i) { fh[4 * b + i] = h[i]; fl[4 * b + i] = lo[i]; }
+            for (int i = 0; i < 4; i += 2) {
+                const v2f16 lo = {_Float16(__builtin_fmaf(acc[b][i], one, -float(h[i]))),
+                                  _Float16(__builtin_fmaf(acc[b][i + 1], one, -float(h[i + 1])))};
+                fh[4 * b + i] = h[i]; fh[4 * b + i + 1] = h[i + 1];
+                fl[4 * b + i] = lo[0]; fl[4 * b + i + 1] = lo[1];
+            }
         }
-        return total;
+        // Radius class 8 reads overlapping pairs of blocks: as one register
+        // tuple the field is used in place (as separate values the compiler
+        // copies every second pair).
+        if constexpr (!G::K48) {
+            typedef uint32_t vregs __attribute__((ext_vector_type(NF / 2)));
+            vregs r = __builtin_bit_cast(vregs, fh), q = __builtin_bit_cast(vregs, fl);
+            asm("" : "+v"(r), "+v"(q));
+            fh = __builtin_bit_cast(vfield, r);
+            fl = __builtin_bit_cast(vfield, q);
+        }
     };
 
     // ------------------------------------------------- horizontal pass
     const bool fast = y0 >= a.fy0 && y0 + 16 <= a.fy1 && x0 >= a.fx0 && x0 + MSTRIP_W <= a.fx1;
-    const int y = y0 + m;
     constexpr int NOUT  = ONE ? 1 : 6;
     constexpr int HL[6] = {ONE ? 1 : 0, 1, 0, 2, 1, 0};   // horizontal table of output k
     constexpr int VL[6] = {0, 0, 1, 0, 1, 2};             // vertical field of output k
-    auto hpass = [&](int k, const vfield& fh, const vfield& fl) {
+    bool hooked = false;                        // uniform
+    const auto hook = [&] {
+        if (!hooked) before_store();
+        hooked = true;
+    };
+    auto hpass = [&](int l, int k, const vfield& fh, const vfield& fl) {
         const int h = HL[k], v = VL[k];
         v4f32 acc[MNB];
 #pragma unroll
@@ -782,46 +1018,104 @@ mfma_compute(const A& a, int y0, int x0, MfmaRaw<IN>& raw, const MfmaTabs& T, fl
             sink(k, acc, u);
             return;
         }
-        if (fast) {
-            // Through the wave's LDS staging area, so that each store writes
-            // 4 rows x 64 contiguous pixels instead of 16 rows x 16.
+        // Through the wave's LDS staging area, in the output's type, so that
+        // each store writes RPI rows x 64 contiguous pixels, 16 bytes a lane
+        // (from the accumulators a store would write 16 rows x 16 pixels).
+        using ST = MStage<OUT>;
+        char* const sb = reinterpret_cast<char*>(stage);
 #pragma unroll
-            for (int o = 0; o < MNB; ++o)
-                *reinterpret_cast<v4f32*>(stage + m * MOPITCH + 16 * o + 4 * g) = acc[o] * u;
-            __builtin_amdgcn_wave_barrier();
-            if constexpr (CPOL == CPOL_NT) {
-#pragma unroll
-                for (int o = 0; o < MNB; ++o) {
-                    const int row = 4 * o + g;
-                    const v4f32 q = *reinterpret_cast<const v4f32*>(stage + row * MOPITCH + 4 * m);
-                    const gptr<OUT> p = reinterpret_cast<gptr<OUT>>(
-                        a.obase[k] + uintptr_t(int64_t(y0 + row) * a.ostride[k] + x0 + 4 * m) * sizeof(OUT));
-                    Px<OUT>::st4nt(p, q[0], q[1], q[2], q[3]);    // written once: streaming stores
-                }
-            } else {
-                // buffer stores carry the cache policy: rows from the strip's
-                // first row (a uniform base), lane offsets in 32 bits (the host
-                // keeps 16 rows of every output within 2^31 bytes, or no strip
-                // takes this path)
-                const __amdgpu_buffer_rsrc_t orsrc = __builtin_amdgcn_make_buffer_rsrc(
-                    reinterpret_cast<void*>(a.obase[k] + uintptr_t(int64_t(y0) * a.ostride[k]) * sizeof(OUT)),
-                    short(0), int(-1), BUF_DWORD3);
-#pragma unroll
-                for (int o = 0; o < MNB; ++o) {
-                    const int row = 4 * o + g;
-                    const v4f32 q = *reinterpret_cast<const v4f32*>(stage + row * MOPITCH + 4 * m);
-                    const uint32_t off = uint32_t((row * a.ostride[k] + x0 + 4 * m) * int(sizeof(OUT)));
-                    Px<OUT>::template st4buf<CPOL>(orsrc, off, q[0], q[1], q[2], q[3]);
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-        } else {
-            const int rv = a.r[v], rh = a.r[h];
-#pragma unroll
-            for (int o = 0; o < MNB; ++o)
-                store4<OUT>(a, k, false, rv, a.nrow - rv, rh, a.ncol - rh, y, x0 + 16 * o + 4 * g,
-                            acc[o][0] * u, acc[o][1] * u, acc[o][2] * u, acc[o][3] * u);
+        for (int o = 0; o < MNB; ++o) {
+            const v4f32 r = acc[o] * u;
+            Px<OUT>::pack4(sb + m * ST::PITCH + (16 * o + 4 * g) * ST::ES, r[0], r[1], r[2], r[3]);
         }
+        if (k == (l == 0 ? 0 : l == 1 ? 2 : 5)) hook();
+        __builtin_amdgcn_wave_barrier();
+        const int r0 = lane / ST::LPR, c0 = lane % ST::LPR * ST::EPL;
+        const char* const src = sb + r0 * ST::PITCH + c0 * ST::ES;
+        // Buffer stores carry the cache policy: rows from the strip's first row
+        // (a uniform base), lane offsets in 32 bits (the host keeps 16 rows of
+        // every output within 2^31 bytes).  No scalar offset: after a 16-byte
+        // store with one the compiler lets the next vector instruction
+        // overwrite the data, and some lanes then stored the new value.
+        // At the edge of the valid region a lane whose pixels all lie outside
+        // takes an offset past the buffer, which drops its store, and the few
+        // chunks an edge cuts store in pieces.  Edge strips keep the policy of
+        // the others where no chunk is cut: lines left dirty in L2 by ordinary
+        // stores are written back when the kernel ends (3840 x 2160 f32 six
+        // outputs: 54.7 us with ordinary stores in the edge strips, 49.6 so).
+        // With a chunk cut (radii that are not a multiple of the chunk), the
+        // streaming pieces of a line cost more than that (256 images of mixed
+        // radii, f32: 1.30 against 1.20 ms).
+        // Float rows that are not aligned to 16 bytes take ordinary stores:
+        // where two strips of a row meet in a cache line, L2 then merges their
+        // parts (3001 x 4003 f32 six outputs: 144 us against 168 streaming).
+        const int pitch = a.ostride[k] * ST::ES;
+        const uintptr_t base = a.obase[k] + uintptr_t(int64_t(y0) * pitch + int64_t(x0) * ST::ES);
+        const int rv = a.r[v], rh = a.r[h];
+        const int x = x0 + c0, xa = rh - x, xb = a.ncol - rh - x;          // valid pixels of the chunk: [xa, xb)
+        if ((ST::ES == 4 || a.aligned) && !a.far) {
+            const __amdgpu_buffer_rsrc_t orsrc =
+                __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base), short(0), 0x7fffffff, BUF_DWORD3);
+            const auto store = [&](auto cp) {
+                constexpr int CP = cp;
+                const int off = r0 * pitch + c0 * ST::ES;
+                if (fast) {
+#pragma unroll
+                    for (int i = 0; i < ST::NI; ++i)
+                        __builtin_amdgcn_raw_buffer_store_b128(
+                            *reinterpret_cast<const v4u32*>(src + i * ST::RPI * ST::PITCH), orsrc, off + i * ST::RPI * pitch, 0, CP);
+                } else {
+                    const int lo = max(xa, 0), hi = min(xb, ST::EPL);
+                    const bool in = lo == 0 && hi == ST::EPL;
+                    unsigned rows = 0;              // row steps inside the valid rows
+#pragma unroll
+                    for (int i = 0; i < ST::NI; ++i) {
+                        const int y = y0 + i * ST::RPI + r0;
+                        rows |= unsigned(y >= rv && y < a.nrow - rv) << i;
+                    }
+                    const bool cut = !in && hi > lo, both = lo > 0 && hi < ST::EPL;
+                    const bool cuts = __builtin_amdgcn_ballot_w64(cut) != 0;
+                    const auto chunks = [&](auto cq) {
+#pragma unroll
+                        for (int i = 0; i < ST::NI; ++i)
+                            __builtin_amdgcn_raw_buffer_store_b128(
+                                *reinterpret_cast<const v4u32*>(src + i * ST::RPI * ST::PITCH), orsrc,
+                                in && (rows >> i & 1u) ? off + i * ST::RPI * pitch : MINVALID, 0, cq);
+                    };
+                    // a cut line is written by two instructions: ordinary stores, which merge
+                    if (!cuts) chunks(std::integral_constant<int, CP>{});
+                    else       chunks(std::integral_constant<int, 0>{});
+                    // cut at one end; a chunk cut at both (an image hardly wider
+                    // than its border) pixel by pixel
+                    if (cuts)
+                        store_cut<ST::ES, 0, ST::NI>(orsrc, src, ST::RPI * ST::PITCH, off, ST::RPI * pitch, lo > 0,
+                                                        cut && !both ? hi - lo : 0, rows);
+                    if (__builtin_amdgcn_ballot_w64(cut && both)) {
+#pragma unroll 1
+                        for (int e = 0; e < ST::EPL; ++e)
+#pragma unroll
+                            for (int i = 0; i < ST::NI; ++i)
+                                store_piece<ST::ES, 1, 0>(
+                                    orsrc, src + e * ST::ES + i * ST::RPI * ST::PITCH,
+                                    cut && both && e >= lo && e < hi && (rows >> i & 1u)
+                                        ? off + e * ST::ES + i * ST::RPI * pitch : MINVALID);
+                    }
+                }
+            };
+            if (ST::ES < 4 || a.aligned) store(std::integral_constant<int, CPOL>{});
+            else                         store(std::integral_constant<int, 0>{});
+        } else {
+            // 16-bit and 8-bit rows that are not aligned to four pixels, rows
+            // too far apart: plain addresses, ordinary stores
+#pragma unroll
+            for (int i = 0; i < ST::NI; ++i) {
+                const int row = i * ST::RPI + r0, y = y0 + row;
+                if (y < rv || y >= a.nrow - rv) continue;
+                const v4u32 q = *reinterpret_cast<const v4u32*>(src + i * ST::RPI * ST::PITCH);
+                store_chunk<ST::ES>(base + uintptr_t(int64_t(row) * pitch + c0 * ST::ES), q, xa, xb);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
 #ifdef TUCU_TIMELINE
         if constexpr (CPOL == CPOL_NT_WT && MODE == MODE_GAUSS && RC == 16 && std::is_same_v<IN, float> &&
                       std::is_same_v<OUT, float>)
@@ -832,49 +1126,50 @@ mfma_compute(const A& a, int y0, int x0, MfmaRaw<IN>& raw, const MfmaTabs& T, fl
     // One field at a time, each followed by the outputs it feeds, so that
     // the first stores leave after a third of the vertical work.
     const unsigned fneed[3] = {ONE ? 1u : mask & 0x0bu, ONE ? 0u : mask & 0x14u, ONE ? 0u : mask & 0x20u};
-    bool check = CHECK;                         // the first field computed vets the strip's input
 #pragma unroll
     for (int l = 0; l < 3; ++l) {
         if (!fneed[l]) continue;
         vfield fh, fl;
-        const float total = vpass(l, fh, fl, check);
-        if (check) {
-            check = false;
-            redo |= __builtin_amdgcn_ballot_w64(!(__builtin_fabsf(total) <= 3.0e38f)) != 0;
-        }
+        vpass(l, fh, fl);
+        if (!(mask >> (l == 0 ? 0 : l == 1 ? 2 : 5) & 1u)) hook();   // else in the field's first output
 #pragma unroll
         for (int k = 0; k < NOUT; ++k)
-            if (VL[k] == l && (mask >> k & 1u)) hpass(k, fh, fl);
+            if (VL[k] == l && (mask >> k & 1u)) hpass(l, k, fh, fl);
     }
     // Rare: the products could not carry this strip's input.  Its outputs are
     // written again by the FP32 form, after the stores above have completed.
     if constexpr (CHECK) {
-        if (redo) {
+        if (p.redo) {                           // wave-uniform
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-            mfma_strip_fp32<RC, IN, OUT, MODE>(a, y0, x0, T, stage, mask);
+            mfma_strip_fp32<RC, IN, OUT, MODE>(opaque_args(a), y0, x0, T, stage, mask);
         }
     }
 }
 
 // The same without a sink, for the outputs of a.mask (every mode that
 // writes its outputs).
-template <int RC, class IN, class OUT, int MODE = MODE_GAUSS, int CPOL = CPOL_NT, bool FRESH = false, class A, class F>
+template <int RC, class IN, class OUT, int MODE = MODE_GAUSS, int CPOL = CPOL_NT, bool FRESH = false, class A, class H>
 __device__ __forceinline__ void
-mfma_compute(const A& a, int y0, int x0, MfmaRaw<IN>& raw, const MfmaTabs& T, float* stage, F&& after_vpass)
+mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const MfmaTabs& T, float* stage, H&& before_store)
 {
-    mfma_compute<RC, IN, OUT, MODE, CPOL, FRESH>(a, y0, x0, raw, T, stage, after_vpass, 0, a.mask);
+    mfma_filter<RC, IN, OUT, MODE, CPOL, FRESH>(a, y0, x0, p, T, stage, 0, a.mask, before_store);
 }
 #undef TUCU_MFMA
 
 // Workgroup tiles (strip-major: tile = tx * tiles_y + ty) hold WY strips
 // down by 4 / WY across, i.e. 16 WY rows x 256 / WY columns.  Every shape
 // filters the same 16 x 64 strips (at rows cy0 + 16 i, columns cx0 + 64 j),
-// so the shape changes no result.  Position of this wave's strip in `tile`;
-// false if the strip lies outside the region.
-template <int WY, class A>
-__device__ __forceinline__ bool mfma_strip_pos(const A& a, int tile, int& y0, int& x0)
+// so the shape changes no result.
+struct TilePos {
+    int ty, tx;                 // first row and column of the tile
+    int y0, x0;                 // first row and column of this wave's strip
+    bool live;                  // the strip lies in the region
+};
+
+template <int WY, int NW = MWAVES, class A>
+__device__ __forceinline__ TilePos mfma_tile_pos(const A& a, int tile)
 {
-    constexpr int WX = MWAVES / WY;
+    constexpr int WX = NW / WY;
     const int tx = tile / a.tiles_y;
     const int ty = tile - tx * a.tiles_y;
     const int w  = int(threadIdx.x) >> 6;
@@ -882,9 +1177,26 @@ __device__ __forceinline__ bool mfma_strip_pos(const A& a, int tile, int& y0, in
     // strip's position is a scalar branch: a divergent if / else around the
     // loads makes the compiler wait for the loads already in flight before
     // the other side's address arithmetic
-    y0 = __builtin_amdgcn_readfirstlane(a.cy0 + ty * (16 * WY) + 16 * (w / WX));
-    x0 = __builtin_amdgcn_readfirstlane(a.cx0 + tx * (MSTRIP_W * WX) + MSTRIP_W * (w % WX));
-    return y0 < a.cy1 && x0 < a.cx1;
+    TilePos p;
+    p.ty = __builtin_amdgcn_readfirstlane(a.cy0 + ty * (16 * WY));
+    p.tx = __builtin_amdgcn_readfirstlane(a.cx0 + tx * (MSTRIP_W * WX));
+    p.y0 = __builtin_amdgcn_readfirstlane(p.ty + 16 * (w / WX));
+    p.x0 = __builtin_amdgcn_readfirstlane(p.tx + MSTRIP_W * (w % WX));
+    p.live = p.y0 < a.cy1 && p.x0 < a.cx1;
+    return p;
+}
+
+// The operands of a strip of the tile whose window, laid out for radius class
+// WC >= RC, is in LDS at win.
+template <int RC, int SY, int SX, class IN, bool FRESH = false, int WC = RC, class A>
+__device__ __forceinline__ void mfma_ops_tile(const A& a, const char* win, MfmaOps& p)
+{
+    using W = MWin<WC, SY, SX, IN>;
+    const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+    int lane = threadIdx.x & 63;
+    if constexpr (FRESH) asm volatile("" : "+v"(lane));    // as for mfma_load
+    mfma_ops_win<RC, IN, W::PITCH>(a, win + (16 * (w / SX) + WC - RC) * W::PITCH + (MSTRIP_W * (w % SX) + WC - RC) * W::ES,
+                                    lane, p);
 }
 
 // First tile of XCD x's range when ntiles tiles are shared by grid
@@ -917,7 +1229,7 @@ __device__ __forceinline__ void mfma_args_early(const A& a)
 // One image, one workgroup per tile (images with no more tiles than
 // resident workgroups, such as 1080p).
 template <int RC, int WY, class IN, class OUT, int MODE = MODE_GAUSS>
-__global__ void __launch_bounds__(64 * MWAVES) __attribute__((amdgpu_waves_per_eu(MFMA_WAVES_PER_SIMD<IN>)))
+__global__ void __launch_bounds__(64 * MWAVES) __attribute__((amdgpu_waves_per_eu(MFMA_WAVES_PER_SIMD)))
 sepfir_mfma_kernel(const SepArgs a)
 {
     __shared__ MfmaTabs T;
@@ -936,20 +1248,35 @@ sepfir_mfma_kernel(const SepArgs a)
 #endif
     stamp(0);
     mfma_args_early(a);
-    int y0, x0;
-    const bool live = mfma_strip_pos<WY>(a, xcd_remap(blockIdx.x, gridDim.x), y0, x0);
-    MfmaRaw<IN> raw;
-    if (live) mfma_load<RC, IN>(a, y0, x0, raw);    // in flight while the tables are built
-    stamp(10);
-    mfma_get_tabs<MODE>(a, T);
-    stamp(11);
-    __syncthreads();
-    stamp(1);
-    if (!live) return;
+    float* const stage = reinterpret_cast<float*>(stage4) + (threadIdx.x >> 6) * 16 * MOPITCH;
+    const TilePos t = mfma_tile_pos<WY>(a, xcd_remap(blockIdx.x, gridDim.x));
+    MfmaOps p;
+    if constexpr (sizeof(IN) < 4) {
+        using W = MWin<RC, WY, MWAVES / WY, IN>;
+        __shared__ v4u32 win4[W::BYTES / 16];
+        char* const win = reinterpret_cast<char*>(win4);
+        v4u32 v[W::N];
+        const int tid = int(threadIdx.x);
+        mwin_load<RC, WY, MWAVES / WY, IN>(a, tid, t.ty, t.tx, v);    // in flight while the tables are copied
+        mfma_get_tabs<MODE>(a, T);
+        mwin_store<RC, WY, MWAVES / WY, IN>(tid, win, v);
+        __syncthreads();
+        if (!t.live) return;
+        mfma_ops_tile<RC, WY, MWAVES / WY, IN>(a, win, p);
+    } else {
+        MfmaRaw raw;
+        if (t.live) mfma_load<RC>(a, t.y0, t.x0, raw);    // in flight while the tables are built
+        stamp(10);
+        mfma_get_tabs<MODE>(a, T);
+        stamp(11);
+        __syncthreads();
+        stamp(1);
+        if (!t.live) return;
+        mfma_ops_raw<RC>(a, raw, p);
+        stamp(2);
+    }
     // one round of workgroups: outputs written through L2 (CPOL_NT_WT)
-    mfma_compute<RC, IN, OUT, MODE, CPOL_NT_WT>(a, y0, x0, raw, T,
-                                                reinterpret_cast<float*>(stage4) + (threadIdx.x >> 6) * 16 * MOPITCH,
-                                                [&] { stamp(2); });
+    mfma_filter<RC, IN, OUT, MODE, CPOL_NT_WT>(a, t.y0, t.x0, p, T, stage, [] {});
     stamp(9);
 }
 
@@ -963,7 +1290,7 @@ sepfir_mfma_kernel(const SepArgs a)
 // them.  (A 4096 x 4096 FIRFilter2 launch: 21.5 us against 25.5 us with one
 // workgroup per tile, which rebuilds the tables 4096 times.)
 template <int RC, int WY, class IN, class OUT, int MODE = MODE_GAUSS>
-__global__ void __launch_bounds__(64 * MWAVES) __attribute__((amdgpu_waves_per_eu(MFMA_LOOP_WAVES<MODE, IN>)))
+__global__ void __launch_bounds__(64 * MWAVES) __attribute__((amdgpu_waves_per_eu(MFMA_LOOP_WAVES<IN>)))
 sepfir_mfma_loop_kernel(const SepArgs a, int ntiles)
 {
     __shared__ MfmaTabs T;
@@ -974,12 +1301,7 @@ sepfir_mfma_loop_kernel(const SepArgs a, int ntiles)
     const int hi = mfma_share_lo(ntiles, grid, x + 1);
     int t = mfma_share_lo(ntiles, grid, x) + b / QN;
     float* const stage = reinterpret_cast<float*>(stage4) + (threadIdx.x >> 6) * 16 * MOPITCH;
-    int y0, x0;
-    bool live = t < hi && mfma_strip_pos<WY>(a, t, y0, x0);
-    MfmaRaw<IN> raw;
-    if (live) mfma_load<RC, IN>(a, y0, x0, raw);    // in flight while the tables are built
-    mfma_get_tabs<MODE>(a, T);
-    __syncthreads();
+    if (t >= hi) return;                            // uniform over the workgroup
     // The six-output strip code for float input takes its lane index afresh
     // in each tile: left to itself the compiler computes the lane-derived
     // offsets once, before the loop, and holds them through it (3840 x 2160
@@ -987,12 +1309,51 @@ sepfir_mfma_loop_kernel(const SepArgs a, int ntiles)
     // and u8 input at radius class 8 3.5 % slower (its registers then fit
     // three waves per SIMD, and the grid, the resident workgroups, grew by
     // half): they keep the hoisted offsets.
-    constexpr bool FRESH = MODE == MODE_GAUSS && sizeof(IN) == 4;
-    while (t < hi) {                                // uniform over the workgroup
-        if (live) mfma_compute<RC, IN, OUT, MODE, CPOL_NT, FRESH>(a, y0, x0, raw, T, stage, [] {});
-        t += step;
-        live = t < hi && mfma_strip_pos<WY>(a, t, y0, x0);
-        if (live) mfma_load<RC, IN, FRESH>(a, y0, x0, raw);
+    constexpr bool FRESH = MODE == MODE_GAUSS || sizeof(IN) < 4;
+    TilePos pos = mfma_tile_pos<WY>(a, t);
+    if constexpr (sizeof(IN) < 4) {
+        using W = MWin<RC, WY, MWAVES / WY, IN>;
+        __shared__ v4u32 win4[W::BYTES / 16];
+        char* const win = reinterpret_cast<char*>(win4);
+        v4u32 v[W::N];
+        int tid = int(threadIdx.x);
+        mwin_load<RC, WY, MWAVES / WY, IN>(a, tid, pos.ty, pos.tx, v);    // in flight while the tables are copied
+        mfma_get_tabs<MODE>(a, T);
+        mwin_store<RC, WY, MWAVES / WY, IN>(tid, win, v);
+        for (;;) {
+            if constexpr (FRESH) asm volatile("" : "+v"(tid));
+            lds_barrier();                          // the window (at first also the tables) is complete
+            MfmaOps p;
+            if (pos.live) mfma_ops_tile<RC, WY, MWAVES / WY, IN, FRESH>(a, win, p);
+            lds_barrier();                          // every wave has its operands: the window may be overwritten
+            const TilePos now = pos;
+            t += step;
+            const bool more = t < hi;
+            if (more) {                             // the next window's loads run under this tile's work
+                pos = mfma_tile_pos<WY>(a, t);
+                mwin_load<RC, WY, MWAVES / WY, IN>(a, tid, pos.ty, pos.tx, v);
+            }
+            const auto next = [&] { if (more) mwin_store<RC, WY, MWAVES / WY, IN>(tid, win, v); };
+            if (now.live) mfma_filter<RC, IN, OUT, MODE, CPOL_NT, FRESH>(a, now.y0, now.x0, p, T, stage, next);
+            else          next();
+            if (!more) break;
+        }
+    } else {
+        MfmaRaw raw;
+        if (pos.live) mfma_load<RC>(a, pos.y0, pos.x0, raw);    // in flight while the tables are built
+        mfma_get_tabs<MODE>(a, T);
+        __syncthreads();
+        while (t < hi) {                            // uniform over the workgroup
+            if (pos.live) {
+                MfmaOps p;
+                mfma_ops_raw<RC>(a, raw, p);
+                mfma_filter<RC, IN, OUT, MODE, CPOL_NT, FRESH>(a, pos.y0, pos.x0, p, T, stage, [] {});
+            }
+            t += step;
+            if (t >= hi) break;
+            pos = mfma_tile_pos<WY>(a, t);
+            if (pos.live) mfma_load<RC, FRESH>(a, pos.y0, pos.x0, raw);
+        }
     }
 }
 
@@ -1026,16 +1387,19 @@ hipError_t launch_sepfir_mfma(const SepArgs& a, int nblocks, hipStream_t s)
 // one-round kernel gets one workgroup per such tile (1080p 17 x 17 lobes,
 // 1 x 4 strips: 7.0 against 7.3 us with 2 x 2); a larger one the tile loop
 // with WYL (the 4096^2 u8 launches 3-7 % slower with 1 x 4 than with 2 x 2).
-template <int RC, int WYR, int WYL, class IN, class OUT>
+// Unaligned rows take WYU.
+template <int RC, int WYR, int WYL, int WYU, class IN, class OUT>
 hipError_t launch_fir_mfma(const SepArgs& a, int nblocks, hipStream_t s)
 {
+    const auto tiles = [&](int wy, SepArgs& r) {
+        r.tiles_y = (a.cy1 - a.cy0 + 16 * wy - 1) / (16 * wy);
+        return int64_t((a.cx1 - a.cx0 + MSTRIP_W * (MWAVES / wy) - 1) / (MSTRIP_W * (MWAVES / wy))) * r.tiles_y;
+    };
+    SepArgs r = a;
+    if (!a.aligned) return launch_sepfir_mfma<RC, WYU, IN, OUT, MODE_TAPS>(r, int(tiles(WYU, r)), s);
     static const int resident = mfma_resident(sepfir_mfma_kernel<RC, WYR, IN, OUT, MODE_TAPS>);
-    const int ty = (a.cy1 - a.cy0 + 16 * WYR - 1) / (16 * WYR);
-    const int tx = (a.cx1 - a.cx0 + MSTRIP_W * (MWAVES / WYR) - 1) / (MSTRIP_W * (MWAVES / WYR));
-    const int64_t n = int64_t(ty) * tx;
+    const int64_t n = tiles(WYR, r);
     if (n > 0 && n <= resident) {
-        SepArgs r = a;
-        r.tiles_y = ty;
         hipLaunchKernelGGL((sepfir_mfma_kernel<RC, WYR, IN, OUT, MODE_TAPS>), dim3(int(n)), dim3(64 * MWAVES), 0, s,
                            r);
         return hipGetLastError();
@@ -1045,17 +1409,15 @@ hipError_t launch_fir_mfma(const SepArgs& a, int nblocks, hipStream_t s)
 
 // Matrix-core variant of batch_kernel: the same tile queue; the tap
 // tables in LDS are rebuilt when the job changes (tiles of a job are
-// contiguous in the list).
-template <int WY, class IN, class OUT>
-__global__ void __launch_bounds__(64 * MWAVES) __attribute__((amdgpu_waves_per_eu(MFMA_WAVES_PER_SIMD<IN>)))
-batch_mfma_kernel(const SepArgs* __restrict__ jobs_, const BatchTile* __restrict__ tiles, int ntiles,
-                  int* __restrict__ counter)
+// contiguous in the list).  Tiles hold SY x SX strips, one per wave (SY = SX
+// = 1: one-wave workgroups, each with its own tables).
+// Float input: each tile is loaded, filtered and stored in turn.
+template <int SY, int SX, class IN, class OUT>
+__device__ __forceinline__ void
+batch_mfma_float(const SepArgs* __restrict__ jobs_, const BatchTile* __restrict__ tiles, int ntiles,
+                 int* __restrict__ counter, MfmaTabs& T, float* stage, int& next)
 {
-    __shared__ MfmaTabs T;
-    __shared__ v4f32 stage4[MWAVES * 16 * MOPITCH / 4];
-    __shared__ int next;
     ConstArgs* const jobs = (ConstArgs*)(uintptr_t)jobs_;
-    float* const stage = reinterpret_cast<float*>(stage4) + (threadIdx.x >> 6) * 16 * MOPITCH;
     int cur = -1;
     TileQueue q;
     int ti = q.first(ntiles);
@@ -1070,16 +1432,18 @@ batch_mfma_kernel(const SepArgs* __restrict__ jobs_, const BatchTile* __restrict
                 cur = int(e.job);
                 __syncthreads();
             }
-            int y0, x0;
-            if (mfma_strip_pos<WY>(a, int(e.tile), y0, x0)) {
-                MfmaRaw<IN> raw;
-                if (a.rt <= 8) {
-                    mfma_load<8, IN>(a, y0, x0, raw);
-                    mfma_compute<8, IN, OUT>(a, y0, x0, raw, T, stage, [] {});
-                } else {
-                    mfma_load<16, IN>(a, y0, x0, raw);
-                    mfma_compute<16, IN, OUT>(a, y0, x0, raw, T, stage, [] {});
-                }
+            const TilePos t = mfma_tile_pos<SY, SY * SX>(a, int(e.tile));
+            if (t.live) {
+                MfmaRaw raw;
+                const auto strip = [&](auto rc) {
+                    constexpr int RC = rc;
+                    MfmaOps p;
+                    mfma_load<RC>(a, t.y0, t.x0, raw);
+                    mfma_ops_raw<RC>(a, raw, p);
+                    mfma_filter<RC, IN, OUT>(a, t.y0, t.x0, p, T, stage, [] {});
+                };
+                if (a.rt <= 8) strip(std::integral_constant<int, 8>{});
+                else           strip(std::integral_constant<int, 16>{});
             }
         }
         __syncthreads();               // T reuse; `next` was written before this barrier
@@ -1089,69 +1453,92 @@ batch_mfma_kernel(const SepArgs* __restrict__ jobs_, const BatchTile* __restrict
     }
 }
 
-// Batched, one wave per workgroup: a tile is one strip (16 x 64; tile =
-// tx * tiles_y + ty), every wave draws its own strips from the counter, so
-// the waves of a SIMD drift apart and their loads, matrix work and stores
-// overlap.  Each wave keeps its own tap tables.
-template <class IN, class OUT>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))   // LDS allows no more
-batch_mfma_wave_kernel(const SepArgs* __restrict__ jobs_, const BatchTile* __restrict__ tiles, int ntiles,
-                       int* __restrict__ counter)
+// Narrow input: the window of the next tile is loaded (into registers) while
+// the current one is filtered, so the queue is asked two tiles ahead; its
+// answer is looked at after the tile's work.
+template <int SY, int SX, class IN, class OUT>
+__device__ __forceinline__ void
+batch_mfma_narrow(const SepArgs* __restrict__ jobs_, const BatchTile* __restrict__ tiles, int ntiles,
+                  int* __restrict__ counter, MfmaTabs& T, float* stage, int& next, char* win)
 {
-    __shared__ MfmaTabs T;
-    __shared__ v4f32 stage4[16 * MOPITCH / 4];
     ConstArgs* const jobs = (ConstArgs*)(uintptr_t)jobs_;
+    v4u32 v[MWin<16, SY, SX, IN>::N];
+    int tid = int(threadIdx.x);
+    int job = 0;                       // of the tile whose window is in v, then in LDS
+    TilePos t{};
+    // one window layout for both radius classes
+    const auto load = [&](int i) {
+        job = __builtin_amdgcn_readfirstlane(int(tiles[i].job));
+        ConstArgs& a = jobs[job];
+        t = mfma_tile_pos<SY, SY * SX>(a, __builtin_amdgcn_readfirstlane(int(tiles[i].tile)));
+        mwin_load<16, SY, SX, IN>(a, tid, t.ty, t.tx, v);
+    };
     int cur = -1;
     TileQueue q;
-    int ti = q.first(ntiles);
-    for (;;) {
-        int nxt = 0;
-        if (threadIdx.x == 0)          // the answer is read after this strip
-            nxt = q.grab(counter, ntiles);
-        if (ti >= 0) {
-            const BatchTile e = tiles[ti];
-            ConstArgs& a = jobs[e.job];
-            if (int(e.job) != cur) {   // one wave: its barrier orders its LDS accesses
-                mfma_build_tabs(a, T);
-                cur = int(e.job);
-                __syncthreads();
-            }
-            const int tx = int(e.tile) / a.tiles_y;
-            const int y0 = __builtin_amdgcn_readfirstlane(a.cy0 + 16 * (int(e.tile) - tx * a.tiles_y));
-            const int x0 = __builtin_amdgcn_readfirstlane(a.cx0 + MSTRIP_W * tx);
-            if (y0 < a.cy1 && x0 < a.cx1) {
-                MfmaRaw<IN> raw;
-                float* const st = reinterpret_cast<float*>(stage4);
-                if (a.rt <= 8) {
-                    mfma_load<8, IN>(a, y0, x0, raw);
-                    mfma_compute<8, IN, OUT>(a, y0, x0, raw, T, st, [] {});
-                } else {
-                    mfma_load<16, IN>(a, y0, x0, raw);
-                    mfma_compute<16, IN, OUT>(a, y0, x0, raw, T, st, [] {});
-                }
-            }
+    const int first = q.first(ntiles);
+    if (threadIdx.x == 0) next = q.grab(counter, ntiles);
+    if (first >= 0) {
+        load(first);
+        mwin_store<16, SY, SX, IN>(tid, win, v);
+    }
+    for (;;) {                         // everything but v, tid and raw is uniform over the workgroup
+        asm volatile("" : "+v"(tid));  // what derives from it is computed in each tile, not held through the loop
+        job = __builtin_amdgcn_readfirstlane(job);
+        ConstArgs& a = jobs[job];
+        if (job != cur) {
+            lds_barrier();             // no wave reads the old tables any more
+            mfma_build_tabs(a, T);
+            cur = job;
         }
-        __builtin_amdgcn_wave_barrier();
-        ti = __builtin_amdgcn_readfirstlane(nxt);
-        if (ti >= ntiles) break;
+        lds_barrier();                 // the window, the tables and `next` are written
+        const int nt = __builtin_amdgcn_readfirstlane(next);
+        const TilePos now = t;
+        const bool small = a.rt <= 8;
+        MfmaOps p;
+        if (now.live) {
+            if (small) mfma_ops_tile<8, SY, SX, IN, true, 16>(a, win, p);
+            else       mfma_ops_tile<16, SY, SX, IN, true>(a, win, p);
+        }
+        lds_barrier();                 // the window and `next` have been read
+        int raw = 0;
+        if (nt < ntiles) {
+            if (threadIdx.x == 0) raw = q.ask(counter);
+            load(nt);
+        }
+        const auto after = [&] { if (nt < ntiles) mwin_store<16, SY, SX, IN>(tid, win, v); };
+        if (!now.live)  after();
+        else if (small) mfma_filter<8, IN, OUT, MODE_GAUSS, CPOL_NT, true>(a, now.y0, now.x0, p, T, stage, after);
+        else            mfma_filter<16, IN, OUT, MODE_GAUSS, CPOL_NT, true>(a, now.y0, now.x0, p, T, stage, after);
+        if (nt >= ntiles) break;
+        if (threadIdx.x == 0) next = q.answer(counter, ntiles, raw);
     }
 }
 
-template <class IN, class OUT>
-hipError_t launch_batch_mfma_wave(const SepArgs* jobs, const BatchTile* tiles, int ntiles, int* counter,
-                                  int grid, hipStream_t s)
+template <int SY, int SX, class IN, class OUT>
+__global__ void __launch_bounds__(64 * SY * SX)
+__attribute__((amdgpu_waves_per_eu(SY * SX == 1 ? 2 : MFMA_WAVES_PER_SIMD)))   // one-wave: LDS allows no more
+batch_mfma_kernel(const SepArgs* __restrict__ jobs, const BatchTile* __restrict__ tiles, int ntiles,
+                  int* __restrict__ counter)
 {
-    hipLaunchKernelGGL(reset_queue<>, dim3(1), dim3(64), 0, s, counter, grid);
-    hipLaunchKernelGGL((batch_mfma_wave_kernel<IN, OUT>), dim3(grid), dim3(64), 0, s, jobs, tiles, ntiles, counter);
-    return hipGetLastError();
+    __shared__ MfmaTabs T;
+    __shared__ v4f32 stage4[SY * SX * 16 * MOPITCH / 4];
+    __shared__ int next;
+    float* const stage = reinterpret_cast<float*>(stage4) + (threadIdx.x >> 6) * 16 * MOPITCH;
+    if constexpr (sizeof(IN) == 4) {
+        batch_mfma_float<SY, SX, IN, OUT>(jobs, tiles, ntiles, counter, T, stage, next);
+    } else {
+        __shared__ v4u32 win4[MWin<16, SY, SX, IN>::BYTES / 16];
+        batch_mfma_narrow<SY, SX, IN, OUT>(jobs, tiles, ntiles, counter, T, stage, next, reinterpret_cast<char*>(win4));
+    }
 }
 
-template <int WY, class IN, class OUT>
+template <int SY, int SX, class IN, class OUT>
 hipError_t launch_batch_mfma(const SepArgs* jobs, const BatchTile* tiles, int ntiles, int* counter,
                              int grid, hipStream_t s)
 {
     hipLaunchKernelGGL(reset_queue<>, dim3(1), dim3(64), 0, s, counter, grid);
-    hipLaunchKernelGGL((batch_mfma_kernel<WY, IN, OUT>), dim3(grid), dim3(64 * MWAVES), 0, s, jobs, tiles, ntiles, counter);
+    hipLaunchKernelGGL((batch_mfma_kernel<SY, SX, IN, OUT>), dim3(grid), dim3(64 * SY * SX), 0, s, jobs, tiles, ntiles,
+                       counter);
     return hipGetLastError();
 }
 
@@ -1166,6 +1553,12 @@ constexpr int MFMA_WYS[NMWY] = {1, 2, 4};
 // 128 (the 4096^2 u8 launches 2.5-7 % slower with 1 x 4), its one-round
 // launches 1 x 4 (launch_fir_mfma); the ICIA pass 1 x 4 (1080p f32 sigma 3
 // projective 8 %, 3840 x 2160 u8 1-3 % faster, 1080p sigma 2 2 % slower).
+// Rows that are not aligned take 4 x 1 strips (16 x 256 pixels), every kernel:
+// neighbouring strips of a row share the cache line where they meet, and the
+// four of a workgroup write it at about the same time, so that L2 merges it
+// (3001 x 4003 packed f32 six outputs: 119 us against 144 with 1 x 4; bf16 64
+// against 89).
+constexpr int MFMA_WY_UNALIGNED = 0;
 constexpr int MFMA_WY_DEFAULT = 2;
 constexpr int MFMA_WY_ONE = 1;
 constexpr int MFMA_WY_ICIA = 2;

@@ -70,8 +70,9 @@ struct SepArgs {
     uint32_t in_bytes;             // bytes from row 0 to the end of the last row
     int      nrow, ncol;
     int      cy0, cy1, cx0, cx1;   // centre region covered by the grid
-    int      fy0, fy1, fx0, fx1;   // centre rectangle on which every live output is valid and
-                                   // takes aligned 4-element stores (empty if stores are unaligned)
+    int      fy0, fy1, fx0, fx1;   // centre rectangle on which every live output is valid
+    int      aligned;              // every live output takes aligned 4-element stores
+    int      far;                  // 16 rows of an output do not fit 31-bit offsets
     int      tiles_y;              // tiles per column strip
     unsigned mask;                 // FIR: bit 0.  GAUSS: smooth, diffH, diffV, diffHH, diffHV, diffVV
     int      r[3];                 // GAUSS: radius of lobe 0, 1, 2.  FIR: r[0] vertical, r[1] horizontal
@@ -123,10 +124,10 @@ template <> struct Px<float> {
     {
         __builtin_nontemporal_store(v4f32{a, b, c, d}, reinterpret_cast<gptr<v4f32>>(p));
     }
-    template <int CP>
-    static __device__ __forceinline__ void st4buf(__amdgpu_buffer_rsrc_t r, uint32_t off, float a, float b, float c, float d)
+    // four adjacent pixels into LDS
+    static __device__ __forceinline__ void pack4(char* p, float a, float b, float c, float d)
     {
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u32, v4f32{a, b, c, d}), r, int(off), 0, CP);
+        *reinterpret_cast<v4f32*>(p) = v4f32{a, b, c, d};
     }
 };
 
@@ -149,10 +150,10 @@ template <> struct Px<uint8_t> {
     {
         __builtin_nontemporal_store(cvt(a) | cvt(b) << 8 | cvt(c) << 16 | cvt(d) << 24, reinterpret_cast<gptr<uint32_t>>(p));
     }
-    template <int CP>
-    static __device__ __forceinline__ void st4buf(__amdgpu_buffer_rsrc_t r, uint32_t off, float a, float b, float c, float d)
+    // four adjacent pixels into LDS
+    static __device__ __forceinline__ void pack4(char* p, float a, float b, float c, float d)
     {
-        __builtin_amdgcn_raw_buffer_store_b32(cvt(a) | cvt(b) << 8 | cvt(c) << 16 | cvt(d) << 24, r, int(off), 0, CP);
+        *reinterpret_cast<uint32_t*>(p) = cvt(a) | cvt(b) << 8 | cvt(c) << 16 | cvt(d) << 24;
     }
 };
 
@@ -170,10 +171,10 @@ template <> struct Px<f16_t> {
     {
         __builtin_nontemporal_store(v2u32{pack_f16(a, b), pack_f16(c, d)}, reinterpret_cast<gptr<v2u32>>(p));
     }
-    template <int CP>
-    static __device__ __forceinline__ void st4buf(__amdgpu_buffer_rsrc_t r, uint32_t off, float a, float b, float c, float d)
+    // four adjacent pixels into LDS
+    static __device__ __forceinline__ void pack4(char* p, float a, float b, float c, float d)
     {
-        __builtin_amdgcn_raw_buffer_store_b64(v2u32{pack_f16(a, b), pack_f16(c, d)}, r, int(off), 0, CP);
+        *reinterpret_cast<v2u32*>(p) = v2u32{pack_f16(a, b), pack_f16(c, d)};
     }
 };
 
@@ -194,10 +195,10 @@ template <> struct Px<bf16_t> {
     {
         __builtin_nontemporal_store(v2u32{pack_bf16(a, b), pack_bf16(c, d)}, reinterpret_cast<gptr<v2u32>>(p));
     }
-    template <int CP>
-    static __device__ __forceinline__ void st4buf(__amdgpu_buffer_rsrc_t r, uint32_t off, float a, float b, float c, float d)
+    // four adjacent pixels into LDS
+    static __device__ __forceinline__ void pack4(char* p, float a, float b, float c, float d)
     {
-        __builtin_amdgcn_raw_buffer_store_b64(v2u32{pack_bf16(a, b), pack_bf16(c, d)}, r, int(off), 0, CP);
+        *reinterpret_cast<v2u32*>(p) = v2u32{pack_bf16(a, b), pack_bf16(c, d)};
     }
 };
 
@@ -486,7 +487,7 @@ sepfir_tile(const A& a, int tile, float* lds)
 
     // ---------------------------------------------------- horizontal pass
     // Uniform: is every store of this tile valid and vector-aligned?
-    const bool fast = cy >= a.fy0 && cy + TH <= a.fy1 && cx >= a.fx0 && cx + TWO <= a.fx1;
+    const bool fast = a.aligned && cy >= a.fy0 && cy + TH <= a.fy1 && cx >= a.fx0 && cx + TWO <= a.fx1;
     if constexpr (FIR) {
         hpass<RH, TH, PITCH, TWO, 0, true, OUT, TAPS>(a, lds, t, cy, cx, fast);
     } else {

@@ -452,7 +452,7 @@ int tucu_server_create(tucu_server* server, const tucu_server_config* cfg)
     int thi = -1;
     const int fam = batch_family();
     const int rows = cfg->tile_rows > 0 ? cfg->tile_rows
-                                        : batch_entry(fam, BATCH_TH_DEFAULT, cfg->in_dtype, cfg->out_dtype).th;
+                                        : batch_entry(fam, batch_default(fam, cfg->in_dtype, cfg->out_dtype), cfg->in_dtype, cfg->out_dtype).th;
     for (int i = 0; i < NBTH; ++i)
         if (batch_entry(fam, i, cfg->in_dtype, cfg->out_dtype).th == rows &&
             batch_entry(fam, i, cfg->in_dtype, cfg->out_dtype).fn)
