@@ -1049,8 +1049,9 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const MfmaTabs& T, flo
         // Float rows that are not aligned to 16 bytes take ordinary stores:
         // where two strips of a row meet in a cache line, L2 then merges their
         // parts (3001 x 4003 f32 six outputs: 144 us against 168 streaming).
-        const int pitch = a.ostride[k] * ST::ES;
-        const uintptr_t base = a.obase[k] + uintptr_t(int64_t(y0) * pitch + int64_t(x0) * ST::ES);
+        const int64_t pitch64 = int64_t(a.ostride[k]) * ST::ES;
+        const int pitch = int(pitch64);         // wraps only where a.far keeps it unused
+        const uintptr_t base = a.obase[k] + uintptr_t(y0 * pitch64 + int64_t(x0) * ST::ES);
         const int rv = a.r[v], rh = a.r[h];
         const int x = x0 + c0, xa = rh - x, xb = a.ncol - rh - x;          // valid pixels of the chunk: [xa, xb)
         if ((ST::ES == 4 || a.aligned) && !a.far) {
@@ -1112,7 +1113,7 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const MfmaTabs& T, flo
                 const int row = i * ST::RPI + r0, y = y0 + row;
                 if (y < rv || y >= a.nrow - rv) continue;
                 const v4u32 q = *reinterpret_cast<const v4u32*>(src + i * ST::RPI * ST::PITCH);
-                store_chunk<ST::ES>(base + uintptr_t(int64_t(row) * pitch + c0 * ST::ES), q, xa, xb);
+                store_chunk<ST::ES>(base + uintptr_t(row * pitch64 + c0 * ST::ES), q, xa, xb);
             }
         }
         __builtin_amdgcn_wave_barrier();
