@@ -43,7 +43,10 @@ int batch_default(int fam, int in_dt, int out_dt)
 
 // Tile list of `jobs` for the tile shape of e (sets every job's tiles_y):
 // tiles of the larger radius classes first (they cost most; handing them out
-// early shortens the tail), each job's tiles in strip-major order.
+// early shortens the tail), each job's tiles in strip-major order, or row by
+// row where the job's output rows do not start at 128-byte lines: tiles that
+// meet in a line then run at about the same time on one XCD, whose L2 merges
+// their parts of it.
 int make_tiles(std::vector<SepArgs>& jobs, const BatchEntry& e, std::vector<BatchTile>& tiles)
 {
     const int th = e.th;
@@ -56,7 +59,9 @@ int make_tiles(std::vector<SepArgs>& jobs, const BatchEntry& e, std::vector<Batc
         const SepArgs& a = jobs[j];
         const int two = e.tw ? e.tw : NT - 2 * a.rt;
         const int64_t n = int64_t((a.cx1 - a.cx0 + two - 1) / two) * a.tiles_y;
-        for (int64_t t = 0; t < n; ++t) tiles.push_back({uint32_t(j), uint32_t(t)});
+        const int64_t nx = a.tiles_y > 0 ? n / a.tiles_y : 0;
+        for (int64_t t = 0; t < n; ++t)
+            tiles.push_back({uint32_t(j), uint32_t(a.lines ? t : t % nx * a.tiles_y + t / nx)});
     }
     if (tiles.size() >= size_t(INT32_MAX)) return fail(TUCU_ERR_INVALID, "batch too large");
     return TUCU_OK;

@@ -128,18 +128,17 @@ int launch_fir_mfma(SepArgs& a, const float* vt, const float* ht, int rV, int rH
 }
 
 // Workgroup shape of the single-image six-output matrix-core kernel:
-// TUCU_MFMA_ROWS (16, 32 or 64 tile rows) overrides the default (64 rows; 16
-// where an output's rows are not aligned).
-int mfma_wy_index(bool aligned)
+// TUCU_MFMA_ROWS (16, 32 or 64 tile rows) overrides the default (64).
+int mfma_wy_index()
 {
     static const int idx = [] {
         const char* e = std::getenv("TUCU_MFMA_ROWS");
         if (e)
             for (int i = 0; i < NMWY; ++i)
                 if (std::atoi(e) == 16 * MFMA_WYS[i]) return i;
-        return -1;
+        return MFMA_WY_DEFAULT;
     }();
-    return idx >= 0 ? idx : aligned ? MFMA_WY_DEFAULT : MFMA_WY_UNALIGNED;
+    return idx;
 }
 
 int gauss_th_index()
@@ -358,17 +357,19 @@ int finish_args(SepArgs& a, const tucu_image& in, unsigned live, const tucu_imag
         break;                                  // the first live output sets the phase
     }
     a.fy0 = a.fx0 = 0; a.fy1 = in.nrow; a.fx1 = in.ncol;
-    bool aligned = true, near = true;
+    bool aligned = true, lines = true, near = true;
     for (int k = 0; k < 6; ++k) {
         if (!(live & (1u << k))) continue;
         a.fy0 = std::max(a.fy0, rv[k]); a.fy1 = std::min(a.fy1, in.nrow - rv[k]);
         a.fx0 = std::max(a.fx0, rh[k]); a.fx1 = std::min(a.fx1, in.ncol - rh[k]);
         const uintptr_t oes = dtype_size(outs[k].dtype);
         if (a.ostride[k] % 4 != 0 || (a.obase[k] + uintptr_t(a.cx0) * oes) % (4 * oes) != 0) aligned = false;
+        if (a.ostride[k] * int64_t(oes) % 128 != 0 || (a.obase[k] + uintptr_t(a.cx0) * oes) % 128 != 0) lines = false;
         // the strips' buffer stores address 16 rows from a strip's first row in 32 bits
         if ((int64_t(16) * a.ostride[k] + in.ncol + 256) * int64_t(oes) >= (int64_t(1) << 31)) near = false;
     }
     a.aligned = aligned;
+    a.lines = lines;
     a.far = !near;
     return TUCU_OK;
 }
@@ -778,7 +779,7 @@ int tucu_gauss2_convolve(const float* lobe0, int n0, const float* lobe1, int n1,
     }
     if (gauss_use_mfma()) {
         const int rc = rmax <= 8 ? 0 : 1;
-        const KernelEntry* m = &g_gauss_mfma_table[rc][mfma_wy_index(a.aligned)][in->dtype][odt];
+        const KernelEntry* m = &g_gauss_mfma_table[rc][mfma_wy_index()][in->dtype][odt];
         if (!m->fn) m = &g_gauss_mfma_table[rc][MFMA_WY_DEFAULT][in->dtype][odt];
         a.tabs = mfma_tabs_for(a, MODE_GAUSS, st);
         return copy.finish(launch(*m, a, st), st);

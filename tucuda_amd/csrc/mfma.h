@@ -296,6 +296,30 @@ store_cut(__amdgpu_buffer_rsrc_t r, const char* src, int rpitch, int at, int opi
     if constexpr (S > 1) store_cut<ES, CPOL, NI, S / 2>(r, src, rpitch, at, opitch, tail, n, rows);
 }
 
+// Stores a strip of float rows that do not start at 128-byte lines, 4 rows an
+// instruction (16 lanes of 16 bytes each), rows pitch bytes apart in the output
+// from base, PITCH in LDS from src (the lane's first chunk, c bytes into row
+// r0): the chunks of whole lines streaming, those of the lines that the strip
+// shares with its neighbours by ordinary stores, which L2 merges.  Streaming a
+// shared line writes it to memory in parts (3001 x 4004 packed f32 six outputs:
+// 142 us), an ordinary store of a whole line leaves it dirty in L2 until it is
+// evicted (100 us); so split 64 us, as rows of whole lines take.
+template <int PITCH>
+__device__ __forceinline__ void
+store_rows(__amdgpu_buffer_rsrc_t r, uintptr_t base, const char* src, int r0, int c, int pitch)
+{
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int at = (r0 + 4 * i) * pitch;
+        const uint32_t seg = uint32_t(base) + uint32_t(at);                     // low bits of the row's address
+        const int f0 = int(-seg & 127u), f1 = 256 - int((seg + 256) & 127u);    // the whole lines of the row
+        const bool whole = c >= f0 && c + 16 <= f1;
+        const v4u32 q = *reinterpret_cast<const v4u32*>(src + 4 * i * PITCH);
+        __builtin_amdgcn_raw_buffer_store_b128(q, r, whole ? at + c : MINVALID, 0, CPOL_NT);
+        __builtin_amdgcn_raw_buffer_store_b128(q, r, whole ? MINVALID : at + c, 0, 0);
+    }
+}
+
 // Input values of field block b for lane (g, m), float input: column x0 - RC +
 // 16 b + m, rows y0 - RC + 8 g + j (j < 8) and, for K = 48, y0 - RC + 32 +
 // 4 g + j (j < 4).  INSIDE: every pixel of the strip's window lies in the
@@ -1046,9 +1070,10 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const MfmaTabs& T, flo
         // With a chunk cut (radii that are not a multiple of the chunk), the
         // streaming pieces of a line cost more than that (256 images of mixed
         // radii, f32: 1.30 against 1.20 ms).
-        // Float rows that are not aligned to 16 bytes take ordinary stores:
-        // where two strips of a row meet in a cache line, L2 then merges their
-        // parts (3001 x 4003 f32 six outputs: 144 us against 168 streaming).
+        // Rows that do not start at 128-byte lines take ordinary stores where
+        // strips meet in a line (store_rows) or, where no line lies within a
+        // strip's row or in a one-round launch, throughout (one-round 1080 x
+        // 1923 f32 16.6 us, split 20.9).
         const int64_t pitch64 = int64_t(a.ostride[k]) * ST::ES;
         const int pitch = int(pitch64);         // wraps only where a.far keeps it unused
         const uintptr_t base = a.obase[k] + uintptr_t(y0 * pitch64 + int64_t(x0) * ST::ES);
@@ -1057,54 +1082,53 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const MfmaTabs& T, flo
         if ((ST::ES == 4 || a.aligned) && !a.far) {
             const __amdgpu_buffer_rsrc_t orsrc =
                 __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base), short(0), 0x7fffffff, BUF_DWORD3);
-            const auto store = [&](auto cp) {
+            const int off = r0 * pitch + c0 * ST::ES;
+            constexpr bool ROWS = ST::ES == 4 && CPOL == CPOL_NT;
+            // row steps of the mask rows, at lanes where in holds
+            const auto chunks = [&](auto cp, bool in, unsigned rows) {
                 constexpr int CP = cp;
-                const int off = r0 * pitch + c0 * ST::ES;
-                if (fast) {
 #pragma unroll
-                    for (int i = 0; i < ST::NI; ++i)
-                        __builtin_amdgcn_raw_buffer_store_b128(
-                            *reinterpret_cast<const v4u32*>(src + i * ST::RPI * ST::PITCH), orsrc, off + i * ST::RPI * pitch, 0, CP);
-                } else {
-                    const int lo = max(xa, 0), hi = min(xb, ST::EPL);
-                    const bool in = lo == 0 && hi == ST::EPL;
-                    unsigned rows = 0;              // row steps inside the valid rows
+                for (int i = 0; i < ST::NI; ++i)
+                    __builtin_amdgcn_raw_buffer_store_b128(
+                        *reinterpret_cast<const v4u32*>(src + i * ST::RPI * ST::PITCH), orsrc,
+                        in && (rows >> i & 1u) ? off + i * ST::RPI * pitch : MINVALID, 0, CP);
+            };
+            const auto streaming = std::integral_constant<int, CPOL>{};
+            const auto ordinary = std::integral_constant<int, 0>{};
+            if (fast) {
+                if (a.lines)   chunks(streaming, true, ~0u);
+                else if (ROWS) store_rows<ST::PITCH>(orsrc, base, src, r0, c0 * ST::ES, pitch);
+                else           chunks(ordinary, true, ~0u);
+            } else {
+                const int lo = max(xa, 0), hi = min(xb, ST::EPL);
+                const bool in = lo == 0 && hi == ST::EPL;
+                unsigned rows = 0;                  // row steps inside the valid rows
 #pragma unroll
-                    for (int i = 0; i < ST::NI; ++i) {
-                        const int y = y0 + i * ST::RPI + r0;
-                        rows |= unsigned(y >= rv && y < a.nrow - rv) << i;
-                    }
-                    const bool cut = !in && hi > lo, both = lo > 0 && hi < ST::EPL;
-                    const bool cuts = __builtin_amdgcn_ballot_w64(cut) != 0;
-                    const auto chunks = [&](auto cq) {
+                for (int i = 0; i < ST::NI; ++i) {
+                    const int y = y0 + i * ST::RPI + r0;
+                    rows |= unsigned(y >= rv && y < a.nrow - rv) << i;
+                }
+                const bool cut = !in && hi > lo, both = lo > 0 && hi < ST::EPL;
+                const bool cuts = __builtin_amdgcn_ballot_w64(cut) != 0;
+                // a cut line is written by two instructions: ordinary stores, which merge
+                if (a.lines && !cuts) chunks(streaming, in, rows);
+                else                  chunks(ordinary, in, rows);
+                // cut at one end; a chunk cut at both (an image hardly wider
+                // than its border) pixel by pixel
+                if (cuts)
+                    store_cut<ST::ES, 0, ST::NI>(orsrc, src, ST::RPI * ST::PITCH, off, ST::RPI * pitch, lo > 0,
+                                                 cut && !both ? hi - lo : 0, rows);
+                if (__builtin_amdgcn_ballot_w64(cut && both)) {
+#pragma unroll 1
+                    for (int e = 0; e < ST::EPL; ++e)
 #pragma unroll
                         for (int i = 0; i < ST::NI; ++i)
-                            __builtin_amdgcn_raw_buffer_store_b128(
-                                *reinterpret_cast<const v4u32*>(src + i * ST::RPI * ST::PITCH), orsrc,
-                                in && (rows >> i & 1u) ? off + i * ST::RPI * pitch : MINVALID, 0, cq);
-                    };
-                    // a cut line is written by two instructions: ordinary stores, which merge
-                    if (!cuts) chunks(std::integral_constant<int, CP>{});
-                    else       chunks(std::integral_constant<int, 0>{});
-                    // cut at one end; a chunk cut at both (an image hardly wider
-                    // than its border) pixel by pixel
-                    if (cuts)
-                        store_cut<ST::ES, 0, ST::NI>(orsrc, src, ST::RPI * ST::PITCH, off, ST::RPI * pitch, lo > 0,
-                                                        cut && !both ? hi - lo : 0, rows);
-                    if (__builtin_amdgcn_ballot_w64(cut && both)) {
-#pragma unroll 1
-                        for (int e = 0; e < ST::EPL; ++e)
-#pragma unroll
-                            for (int i = 0; i < ST::NI; ++i)
-                                store_piece<ST::ES, 1, 0>(
-                                    orsrc, src + e * ST::ES + i * ST::RPI * ST::PITCH,
-                                    cut && both && e >= lo && e < hi && (rows >> i & 1u)
-                                        ? off + e * ST::ES + i * ST::RPI * pitch : MINVALID);
-                    }
+                            store_piece<ST::ES, 1, 0>(
+                                orsrc, src + e * ST::ES + i * ST::RPI * ST::PITCH,
+                                cut && both && e >= lo && e < hi && (rows >> i & 1u)
+                                    ? off + e * ST::ES + i * ST::RPI * pitch : MINVALID);
                 }
-            };
-            if (ST::ES < 4 || a.aligned) store(std::integral_constant<int, CPOL>{});
-            else                         store(std::integral_constant<int, 0>{});
+            }
         } else {
             // 16-bit and 8-bit rows that are not aligned to four pixels, rows
             // too far apart: plain addresses, ordinary stores
@@ -1311,7 +1335,13 @@ sepfir_mfma_loop_kernel(const SepArgs a, int ntiles)
     // three waves per SIMD, and the grid, the resident workgroups, grew by
     // half): they keep the hoisted offsets.
     constexpr bool FRESH = MODE == MODE_GAUSS || sizeof(IN) < 4;
-    TilePos pos = mfma_tile_pos<WY>(a, t);
+    // Output rows that do not start at 128-byte lines: the tiles row by row, so
+    // that tiles which meet in a line run at about the same time and L2 merges
+    // their parts of it (3001 x 4003 packed, radius 16: bf16 66 -> 58 us, f32 91
+    // -> 87 against tiles of 16 x 256 pixels in strip-major order).
+    const int nx = a.lines ? 0 : ntiles / a.tiles_y;
+    const auto place = [&](int i) { return mfma_tile_pos<WY>(a, nx ? i % nx * a.tiles_y + i / nx : i); };
+    TilePos pos = place(t);
     if constexpr (sizeof(IN) < 4) {
         using W = MWin<RC, WY, MWAVES / WY, IN>;
         __shared__ v4u32 win4[W::BYTES / 16];
@@ -1331,7 +1361,7 @@ sepfir_mfma_loop_kernel(const SepArgs a, int ntiles)
             t += step;
             const bool more = t < hi;
             if (more) {                             // the next window's loads run under this tile's work
-                pos = mfma_tile_pos<WY>(a, t);
+                pos = place(t);
                 mwin_load<RC, WY, MWAVES / WY, IN>(a, tid, pos.ty, pos.tx, v);
             }
             const auto next = [&] { if (more) mwin_store<RC, WY, MWAVES / WY, IN>(tid, win, v); };
@@ -1352,7 +1382,7 @@ sepfir_mfma_loop_kernel(const SepArgs a, int ntiles)
             }
             t += step;
             if (t >= hi) break;
-            pos = mfma_tile_pos<WY>(a, t);
+            pos = place(t);
             if (pos.live) mfma_load<RC, FRESH>(a, pos.y0, pos.x0, raw);
         }
     }
@@ -1371,41 +1401,26 @@ int mfma_resident(K kernel)
     return std::max(1, ncu) * per_cu;
 }
 
-template <int RC, int WY, class IN, class OUT, int MODE = MODE_GAUSS>
+// One image in the region of a: one workgroup per WYR-shaped tile where they
+// fit the resident workgroups, else the tile loop with WYL, whose tile count
+// nblocks and tiles_y the call brings.  (One-output launches, MODE_TAPS, WYR =
+// 1 x 4 strips and WYL = 2 x 2: 1080p 17 x 17 lobes 7.0 us against 7.3 with 2 x
+// 2, the 4096^2 u8 launches 3-7 % slower with 1 x 4.)
+template <int RC, int WYR, int WYL, class IN, class OUT, int MODE = MODE_GAUSS>
 hipError_t launch_sepfir_mfma(const SepArgs& a, int nblocks, hipStream_t s)
 {
-    static const int resident = mfma_resident(sepfir_mfma_loop_kernel<RC, WY, IN, OUT, MODE>);
-    if (nblocks <= resident)
-        hipLaunchKernelGGL((sepfir_mfma_kernel<RC, WY, IN, OUT, MODE>), dim3(nblocks), dim3(64 * MWAVES), 0, s, a);
-    else
-        hipLaunchKernelGGL((sepfir_mfma_loop_kernel<RC, WY, IN, OUT, MODE>), dim3(resident), dim3(64 * MWAVES), 0, s,
-                           a, nblocks);
-    return hipGetLastError();
-}
-
-// One-output launches (MODE_TAPS), given the grid of the tile loop's shape
-// WYL: an image whose 16 WYR-row tiles fit the resident workgroups of the
-// one-round kernel gets one workgroup per such tile (1080p 17 x 17 lobes,
-// 1 x 4 strips: 7.0 against 7.3 us with 2 x 2); a larger one the tile loop
-// with WYL (the 4096^2 u8 launches 3-7 % slower with 1 x 4 than with 2 x 2).
-// Unaligned rows take WYU.
-template <int RC, int WYR, int WYL, int WYU, class IN, class OUT>
-hipError_t launch_fir_mfma(const SepArgs& a, int nblocks, hipStream_t s)
-{
-    const auto tiles = [&](int wy, SepArgs& r) {
-        r.tiles_y = (a.cy1 - a.cy0 + 16 * wy - 1) / (16 * wy);
-        return int64_t((a.cx1 - a.cx0 + MSTRIP_W * (MWAVES / wy) - 1) / (MSTRIP_W * (MWAVES / wy))) * r.tiles_y;
-    };
+    static const int loop = mfma_resident(sepfir_mfma_loop_kernel<RC, WYL, IN, OUT, MODE>);
+    static const int one = MODE == MODE_TAPS ? mfma_resident(sepfir_mfma_kernel<RC, WYR, IN, OUT, MODE>) : loop;
+    constexpr int H = 16 * WYR, W = MSTRIP_W * (MWAVES / WYR);
     SepArgs r = a;
-    if (!a.aligned) return launch_sepfir_mfma<RC, WYU, IN, OUT, MODE_TAPS>(r, int(tiles(WYU, r)), s);
-    static const int resident = mfma_resident(sepfir_mfma_kernel<RC, WYR, IN, OUT, MODE_TAPS>);
-    const int64_t n = tiles(WYR, r);
-    if (n > 0 && n <= resident) {
-        hipLaunchKernelGGL((sepfir_mfma_kernel<RC, WYR, IN, OUT, MODE_TAPS>), dim3(int(n)), dim3(64 * MWAVES), 0, s,
-                           r);
-        return hipGetLastError();
-    }
-    return launch_sepfir_mfma<RC, WYL, IN, OUT, MODE_TAPS>(a, nblocks, s);
+    r.tiles_y = (a.cy1 - a.cy0 + H - 1) / H;
+    const int64_t n = int64_t((a.cx1 - a.cx0 + W - 1) / W) * r.tiles_y;
+    if (n <= one)
+        hipLaunchKernelGGL((sepfir_mfma_kernel<RC, WYR, IN, OUT, MODE>), dim3(int(n)), dim3(64 * MWAVES), 0, s, r);
+    else
+        hipLaunchKernelGGL((sepfir_mfma_loop_kernel<RC, WYL, IN, OUT, MODE>), dim3(std::min(nblocks, loop)),
+                           dim3(64 * MWAVES), 0, s, a, nblocks);
+    return hipGetLastError();
 }
 
 // Matrix-core variant of batch_kernel: the same tile queue; the tap
@@ -1552,14 +1567,8 @@ constexpr int MFMA_WYS[NMWY] = {1, 2, 4};
 // 2 x 2, 3840 x 2160 3 %: the strips of a workgroup share their vertical
 // halo rows in L1); the one-output FIR / general-taps tile loop 2 x 2, 32 x
 // 128 (the 4096^2 u8 launches 2.5-7 % slower with 1 x 4), its one-round
-// launches 1 x 4 (launch_fir_mfma); the ICIA pass 1 x 4 (1080p f32 sigma 3
+// launches 1 x 4 (launch_sepfir_mfma); the ICIA pass 1 x 4 (1080p f32 sigma 3
 // projective 8 %, 3840 x 2160 u8 1-3 % faster, 1080p sigma 2 2 % slower).
-// Rows that are not aligned take 4 x 1 strips (16 x 256 pixels), every kernel:
-// neighbouring strips of a row share the cache line where they meet, and the
-// four of a workgroup write it at about the same time, so that L2 merges it
-// (3001 x 4003 packed f32 six outputs: 119 us against 144 with 1 x 4; bf16 64
-// against 89).
-constexpr int MFMA_WY_UNALIGNED = 0;
 constexpr int MFMA_WY_DEFAULT = 2;
 constexpr int MFMA_WY_ONE = 1;
 constexpr int MFMA_WY_ICIA = 2;

@@ -72,6 +72,7 @@ struct SepArgs {
     int      cy0, cy1, cx0, cx1;   // centre region covered by the grid
     int      fy0, fy1, fx0, fx1;   // centre rectangle on which every live output is valid
     int      aligned;              // every live output takes aligned 4-element stores
+    int      lines;                // tile rows of every live output start at 128-byte lines
     int      far;                  // 16 rows of an output do not fit 31-bit offsets
     int      tiles_y;              // tiles per column strip
     unsigned mask;                 // FIR: bit 0.  GAUSS: smooth, diffH, diffV, diffHH, diffHV, diffVV
@@ -101,7 +102,10 @@ typedef const __attribute__((address_space(4))) SepArgs ConstArgs;
 // streaming and at agent scope, so written through the XCD's L2: the
 // kernel-end release then finds no dirty output lines to write back, which
 // takes 4 % off a one-round launch (1080p six outputs) but costs 3-7 % in
-// the tile loops, where the L2 absorbs the stores of many rounds.
+// the tile loops, where the L2 absorbs the stores of many rounds.  (Written
+// through without streaming, outputs stay in the memory-side cache: the same
+// 1080p buffers again 11.1 us against 14.1 at radius 8, but 16 frames one after
+// the other, which it does not hold, 255 us against 236.)
 constexpr int CPOL_NT = 2;
 constexpr int CPOL_NT_WT = 2 | 16;
 
