@@ -54,44 +54,86 @@ __device__ __forceinline__ float row_sum(float v)
     return v;
 }
 
+// w^n as a constant, n = 0 .. 4.
+constexpr float icia_pow(float w, int n) { return n == 0 ? 1.f : w * icia_pow(w, n - 1); }
+constexpr float ICIA_C[5][5] = {{1, 0, 0, 0, 0}, {1, 1, 0, 0, 0}, {1, 2, 1, 0, 0}, {1, 3, 3, 1, 0}, {1, 4, 6, 4, 1}};
+
+// acc += e K, the constant in the instruction (left to the compiler, the 64
+// constants of a strip are hoisted out of the tile loop into registers).
+template <int K> __device__ __forceinline__ void fma_const(float& acc, float e)
+{
+    asm("v_fmamk_f32 %0, %1, %2, %0" : "+v"(acc) : "v"(e), "n"(K));
+}
+
 // mom[k * ms] += the moments of this lane's 16 pixels (row y, columns x0 +
 // 16 o + 4 g + i of the accumulators gH, gV), zero outside each gradient's
-// valid region.
+// valid region.  The vector units bound the pass (2160p u8: 8.3 M pixels), so
+// the pixel loop has no more than the sums need: the powers of a pixel's column
+// are those of w = 16 o + i - 25.5, constants, relative to the lane's column uc,
+// and u^n = (uc + sc w)^n is expanded once per strip; and only strips that
+// meet the border of the valid region mask their pixels.
 template <int D>
-__device__ __forceinline__ void icia_lane_moments(const SepArgs& a, int y0, int x0, const v4f32* gH,
-                                                  const v4f32* gV, float* mom, int ms)
+__device__ __forceinline__ void icia_lane_moments(const SepArgs& a, int y0, int x0, v4f32* gH, v4f32* gV, float* mom,
+                                                  int ms)
 {
     constexpr int NU = D == 6 ? 3 : 5;          // powers of u: 0 .. 2 (affine), 0 .. 4
     const int lane = threadIdx.x & 63, g = lane >> 4, m = lane & 15;
     const float sc = 1.f / float(max(a.nrow, a.ncol));
     const int y = y0 + m, r0 = a.r[0], r1 = a.r[1];
-    const bool rowH = y >= r0 && y < a.nrow - r0;          // diffH: V lobe 0, H lobe 1
-    const bool rowV = y >= r1 && y < a.nrow - r1;          // diffV: V lobe 1, H lobe 0
-    float A[3][NU];
+    const int rr = max(r0, r1);
+    if (!(y0 >= rr && y0 + 16 <= a.nrow - rr && x0 >= rr && x0 + MSTRIP_W <= a.ncol - rr)) {    // uniform
+        const bool rowH = y >= r0 && y < a.nrow - r0;      // diffH: V lobe 0, H lobe 1
+        const bool rowV = y >= r1 && y < a.nrow - r1;      // diffV: V lobe 1, H lobe 0
+#pragma unroll
+        for (int o = 0; o < MNB; ++o)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int x = x0 + 16 * o + 4 * g + i;
+                gH[o][i] = rowH && x >= r1 && x < a.ncol - r1 ? gH[o][i] : 0.f;
+                gV[o][i] = rowV && x >= r0 && x < a.ncol - r0 ? gV[o][i] : 0.f;
+            }
+    }
+    float W[3][NU];                             // sums of e_X e_Y w^n
 #pragma unroll
     for (int xy = 0; xy < 3; ++xy)
 #pragma unroll
-        for (int n = 0; n < NU; ++n) A[xy][n] = 0.f;
+        for (int n = 0; n < NU; ++n) W[xy][n] = 0.f;
+    static_for<0, 4 * MNB>([&](auto pc) {
+        constexpr int o = pc / 4, i = pc % 4;
+        constexpr float w = 16 * o + i - 25.5f;
+        const float eH = gH[o][i], eV = gV[o][i];
+        const float ee[3] = {eH * eH, eH * eV, eV * eV};
 #pragma unroll
-    for (int o = 0; o < MNB; ++o)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int x = x0 + 16 * o + 4 * g + i;
-            const float eH = rowH && x >= r1 && x < a.ncol - r1 ? gH[o][i] : 0.f;
-            const float eV = rowV && x >= r0 && x < a.ncol - r0 ? gV[o][i] : 0.f;
-            const float ee[3] = {eH * eH, eH * eV, eV * eV};
-            float up[NU];
-            up[0] = 1.f;
-            up[1] = sc * float(x);
-#pragma unroll
-            for (int n = 2; n < NU; ++n) up[n] = up[n - 1] * up[1];
-#pragma unroll
-            for (int xy = 0; xy < 3; ++xy) {
-                A[xy][0] += ee[xy];
-#pragma unroll
-                for (int n = 1; n < NU; ++n) A[xy][n] = __builtin_fmaf(ee[xy], up[n], A[xy][n]);
-            }
+        for (int xy = 0; xy < 3; ++xy) {
+            W[xy][0] += ee[xy];
+            static_for<1, NU>([&](auto nc) {
+                constexpr int n = nc;
+                fma_const<__builtin_bit_cast(int, icia_pow(w, n))>(W[xy][n], ee[xy]);
+            });
         }
+    });
+    // A[xy][n] = sum of e_X e_Y (uc + sc w)^n
+    float A[3][NU], up[NU], sp[NU];
+    up[0] = sp[0] = 1.f;
+    up[1] = sc * (float(x0 + 4 * g) + 25.5f);
+    sp[1] = sc;
+#pragma unroll
+    for (int n = 2; n < NU; ++n) {
+        up[n] = up[n - 1] * up[1];
+        sp[n] = sp[n - 1] * sc;
+    }
+#pragma unroll
+    for (int xy = 0; xy < 3; ++xy) {
+#pragma unroll
+        for (int n = 1; n < NU; ++n) W[xy][n] *= sp[n];
+#pragma unroll
+        for (int n = 0; n < NU; ++n) {
+            float s = W[xy][n];
+#pragma unroll
+            for (int k = n - 1; k >= 0; --k) s = __builtin_fmaf(ICIA_C[n][k] * up[n - k], W[xy][k], s);
+            A[xy][n] = s;
+        }
+    }
     float vp[5];
     vp[0] = 1.f;
     vp[1] = sc * float(y);
