@@ -99,12 +99,22 @@ __device__ __forceinline__ void tl_stamp(int i)
 // left side +c[k] and the lower / right side -c[k] (FIRFilter.h:66-176 pairs
 // them the same way).  A lane's operand is one or two runs, so it loads
 // with 8-byte LDS reads and needs no conversion.
-struct alignas(16) MfmaTabs {
-    v4f16 run[2 * 3 * MT4];
-    v8f16 hpair[2 * 3 * MHP];  // horizontal operands: runs t and t + 16 side by side
-    float lobe[2 * 33];        // staging: cv[l][k] at 17 l + k (GAUSS), tv / th at 33 l + o + 16 (TAPS)
-    float tap[3][MT4 + 4];     // staging: tap o of lobe l times mp[l] at [l][o + MBASE]
+// ONE: of a one-output launch, the runs of the vertical taps (lobe 0) and the
+// pairs of the horizontal ones (lobe 1) only: 6 KB instead of 16, which leave a
+// CU's LDS to four workgroups of a tile loop with 16-bit input instead of three
+// and shorten the copy.
+template <bool ONE> struct alignas(16) MfmaTabsOf {
+    static constexpr int NL = ONE ? 1 : 3;
+    v4f16 run[2 * NL * MT4];
+    v8f16 hpair[2 * NL * MHP]; // horizontal operands: runs t and t + 16 side by side
+    float lobe[ONE ? 68 : 66]; // staging: cv[l][k] at 17 l + k (GAUSS), tv / th at 33 l + o + 16 (TAPS)
+    float tap[ONE ? 2 : 3][MT4 + 4];   // staging: tap o of lobe l times mp[l] at [l][o + MBASE]
+
+    static __device__ __forceinline__ int run_at(int part, int l) { return (part * NL + (ONE ? 0 : l)) * MT4; }
+    static __device__ __forceinline__ int pair_at(int part, int l) { return (part * NL + (ONE ? 0 : l)) * MHP; }
 };
+using MfmaTabs = MfmaTabsOf<false>;             // the layout of tables in device memory
+template <int MODE> using ModeTabs = MfmaTabsOf<MODE == MODE_TAPS>;
 
 // f(std::integral_constant<int, I>) for I = 0 .. N-1, unrolled.
 template <int I, int N, class F>
@@ -122,7 +132,7 @@ __device__ __forceinline__ void static_for(F&& f)
 // table 1 the horizontal ones, both as full taps with tap o at index o + 16
 // of tv / th.
 template <int MODE>
-__device__ __forceinline__ float mfma_tap_lds(const MfmaTabs& T, int l, int o)
+__device__ __forceinline__ float mfma_tap_lds(const ModeTabs<MODE>& T, int l, int o)
 {
     const int k = o < 0 ? -o : o;
     if (k > 16) return 0.f;
@@ -143,7 +153,7 @@ template <int MODE> constexpr int mfma_nlobes() { return MODE == MODE_TAPS ? 2 :
 // a strip's input, stay in flight) and written to LDS by one lane; every
 // entry is then built from LDS.
 template <int MODE = MODE_GAUSS, class A>
-__device__ __forceinline__ void mfma_build_tabs(const A& a, MfmaTabs& T)
+__device__ __forceinline__ void mfma_build_tabs(const A& a, ModeTabs<MODE>& T)
 {
     constexpr int NL = mfma_nlobes<MODE>();
     constexpr int NW = MODE == MODE_TAPS ? 66 : 51;
@@ -169,6 +179,7 @@ __device__ __forceinline__ void mfma_build_tabs(const A& a, MfmaTabs& T)
         const int ee = pair ? e - NL * MT4 : e;
         const int n = pair ? MHP : MT4;
         const int l = ee / n, t = ee - l * n;
+        if (MODE == MODE_TAPS && l != int(pair)) continue;
         v8f16 hi, lo;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {               // taps t .. t + 3, then (pairs) t + 16 .. t + 19
@@ -178,11 +189,11 @@ __device__ __forceinline__ void mfma_build_tabs(const A& a, MfmaTabs& T)
             lo[i] = _Float16(c - float(h));
         }
         if (pair) {
-            T.hpair[(0 * 3 + l) * MHP + t] = hi;
-            T.hpair[(1 * 3 + l) * MHP + t] = lo;
+            T.hpair[T.pair_at(0, l) + t] = hi;
+            T.hpair[T.pair_at(1, l) + t] = lo;
         } else {
-            T.run[(0 * 3 + l) * MT4 + t] = __builtin_shufflevector(hi, hi, 0, 1, 2, 3);
-            T.run[(1 * 3 + l) * MT4 + t] = __builtin_shufflevector(lo, lo, 0, 1, 2, 3);
+            T.run[T.run_at(0, l) + t] = __builtin_shufflevector(hi, hi, 0, 1, 2, 3);
+            T.run[T.run_at(1, l) + t] = __builtin_shufflevector(lo, lo, 0, 1, 2, 3);
         }
     }
 }
@@ -193,12 +204,24 @@ __device__ __forceinline__ void mfma_build_tabs(const A& a, MfmaTabs& T)
 // of the workgroup calls it; the caller puts a barrier between it and the
 // first use of T.  (Building them took 2-3 us of a 1080p launch.)
 template <int MODE = MODE_GAUSS, class A>
-__device__ __forceinline__ void mfma_get_tabs(const A& a, MfmaTabs& T)
+__device__ __forceinline__ void mfma_get_tabs(const A& a, ModeTabs<MODE>& T)
 {
     if (a.tabs) {                               // uniform
         const gptr<const v4f32> src = reinterpret_cast<gptr<const v4f32>>(reinterpret_cast<uintptr_t>(a.tabs));
         v4f32* const dst = reinterpret_cast<v4f32*>(&T);
-        for (int i = threadIdx.x; i < int(sizeof(MfmaTabs) / 16); i += blockDim.x) dst[i] = src[i];
+        if constexpr (MODE == MODE_TAPS) {
+            // run (part 0, 1; lobe 0), pair (part 0, 1; lobe 1), lobe words: 16-byte words of either layout
+            constexpr int RN = MT4 / 2, HN = MHP, LN = 17, H0 = 2 * 3 * RN, L0 = H0 + 2 * 3 * HN;
+            static_assert(offsetof(MfmaTabs, hpair) == 16 * H0 && offsetof(MfmaTabs, lobe) == 16 * L0);
+            static_assert(offsetof(ModeTabs<MODE>, hpair) == 32 * RN && offsetof(ModeTabs<MODE>, lobe) == 32 * (RN + HN));
+            for (int i = threadIdx.x; i < 2 * (RN + HN) + LN; i += blockDim.x) {
+                const int h = i - 2 * RN, l = h - 2 * HN;
+                dst[i] = src[l >= 0 ? L0 + l : h >= HN ? H0 + 4 * HN + (h - HN) : h >= 0 ? H0 + HN + h :
+                             i >= RN ? 3 * RN + (i - RN) : i];
+            }
+        } else {
+            for (int i = threadIdx.x; i < int(sizeof(MfmaTabs) / 16); i += blockDim.x) dst[i] = src[i];
+        }
     } else {
         mfma_build_tabs<MODE>(a, T);
     }
@@ -558,7 +581,7 @@ __device__ __forceinline__ float fp32_taps(const C& t, int r, const W& w)
 // nonzero) are c(k) on the upper / left side.
 template <int RC, class IN, class OUT, int MODE>
 __device__ __forceinline__ void
-mfma_strip_fp32(ConstArgs& a, int y0, int x0, const MfmaTabs& T, float* stage, unsigned mask)
+mfma_strip_fp32(ConstArgs& a, int y0, int x0, const ModeTabs<MODE>& T, float* stage, unsigned mask)
 {
     constexpr bool ONE = MODE == MODE_TAPS;
     constexpr int NFC = 32 + 2 * RC;            // field columns per half strip
@@ -908,7 +931,7 @@ __device__ __forceinline__ void mfma_ops_win(const A& a, const char* win, int la
 //     by d = 32 p - 16 o (zero for the block outside the window).
 template <int RC, class IN, class OUT, int MODE = MODE_GAUSS, int CPOL = CPOL_NT, bool FRESH = false, class A, class S, class H>
 __device__ __forceinline__ void
-mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const MfmaTabs& T, float* stage, S&& sink, unsigned mask,
+mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& T, float* stage, S&& sink, unsigned mask,
             H&& before_store)
 {
     constexpr bool ONE = MODE == MODE_TAPS;     // one field (table 0), one output (table 1 across)
@@ -935,13 +958,13 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const MfmaTabs& T, flo
     asm("" : "+v"(one));
     auto vpass = [&](int l, vfield& fh, vfield& fl) {
         const int t1 = MBASE + 8 * g - RC - m;
-        const v8f16 ch1 = cat8(T.run[(0 * 3 + l) * MT4 + t1], T.run[(0 * 3 + l) * MT4 + t1 + 4]);
-        const v8f16 cl1 = cat8(T.run[(1 * 3 + l) * MT4 + t1], T.run[(1 * 3 + l) * MT4 + t1 + 4]);
+        const v8f16 ch1 = cat8(T.run[T.run_at(0, l) + t1], T.run[T.run_at(0, l) + t1 + 4]);
+        const v8f16 cl1 = cat8(T.run[T.run_at(1, l) + t1], T.run[T.run_at(1, l) + t1 + 4]);
         v8f16 cht, clt;
         if constexpr (G::K48) {                 // rows 32 + 4 g + j: high taps for both halves
             const int t2 = MBASE + 32 + 4 * g - RC - m;
-            const v4f16 th = T.run[(0 * 3 + l) * MT4 + t2];
-            const v4f16 tl = T.run[(1 * 3 + l) * MT4 + t2];
+            const v4f16 th = T.run[T.run_at(0, l) + t2];
+            const v4f16 tl = T.run[T.run_at(1, l) + t2];
             cht = XLO ? cat8(th, th) : cat8(th, tl);
             clt = cat8(tl, z4);
         }
@@ -1013,8 +1036,8 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const MfmaTabs& T, flo
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int t = MBASE + 16 * i - 16 + 4 * g - RC - m;
-                ah[i] = T.hpair[(0 * 3 + h) * MHP + t];
-                al[i] = T.hpair[(1 * 3 + h) * MHP + t];
+                ah[i] = T.hpair[T.pair_at(0, h) + t];
+                al[i] = T.hpair[T.pair_at(1, h) + t];
             }
             // smaller products first, as in the vertical pass
             static_for<0, MNB>([&](auto oc) { constexpr int o = oc, p = o / 2, i = (o & 1) ? 0 : 1;
@@ -1031,8 +1054,8 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const MfmaTabs& T, flo
                 acc[o] = TUCU_MFMA(ah[i], pairP<p>(fh), acc[o]); });
         } else {
             const int t1 = MBASE + 4 * g - RC - m;
-            const v8f16 ch1 = T.hpair[(0 * 3 + h) * MHP + t1];
-            const v8f16 cl1 = T.hpair[(1 * 3 + h) * MHP + t1];
+            const v8f16 ch1 = T.hpair[T.pair_at(0, h) + t1];
+            const v8f16 cl1 = T.hpair[T.pair_at(1, h) + t1];
             static_for<0, MNB>([&](auto oc) { constexpr int o = oc; acc[o] = TUCU_MFMA(cl1, pair8<o>(fh), acc[o]); });
             static_for<0, MNB>([&](auto oc) { constexpr int o = oc; acc[o] = TUCU_MFMA(ch1, pair8<o>(fl), acc[o]); });
             static_for<0, MNB>([&](auto oc) { constexpr int o = oc; acc[o] = TUCU_MFMA(ch1, pair8<o>(fh), acc[o]); });
@@ -1175,7 +1198,7 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const MfmaTabs& T, flo
 // writes its outputs).
 template <int RC, class IN, class OUT, int MODE = MODE_GAUSS, int CPOL = CPOL_NT, bool FRESH = false, class A, class H>
 __device__ __forceinline__ void
-mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const MfmaTabs& T, float* stage, H&& before_store)
+mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& T, float* stage, H&& before_store)
 {
     mfma_filter<RC, IN, OUT, MODE, CPOL, FRESH>(a, y0, x0, p, T, stage, 0, a.mask, before_store);
 }
@@ -1257,7 +1280,7 @@ template <int RC, int WY, class IN, class OUT, int MODE = MODE_GAUSS>
 __global__ void __launch_bounds__(64 * MWAVES) __attribute__((amdgpu_waves_per_eu(MFMA_WAVES_PER_SIMD)))
 sepfir_mfma_kernel(const SepArgs a)
 {
-    __shared__ MfmaTabs T;
+    __shared__ ModeTabs<MODE> T;
     __shared__ v4f32 stage4[MWAVES * 16 * MOPITCH / 4];
 #ifdef TUCU_TIMELINE
     constexpr bool TL = MODE == MODE_GAUSS && RC == 16 && std::is_same_v<IN, float> && std::is_same_v<OUT, float>;
@@ -1318,7 +1341,7 @@ template <int RC, int WY, class IN, class OUT, int MODE = MODE_GAUSS>
 __global__ void __launch_bounds__(64 * MWAVES) __attribute__((amdgpu_waves_per_eu(MFMA_LOOP_WAVES<IN>)))
 sepfir_mfma_loop_kernel(const SepArgs a, int ntiles)
 {
-    __shared__ MfmaTabs T;
+    __shared__ ModeTabs<MODE> T;
     __shared__ v4f32 stage4[MWAVES * 16 * MOPITCH / 4];
     mfma_args_early(a);
     const int grid = int(gridDim.x), b = int(blockIdx.x);
@@ -1330,11 +1353,15 @@ sepfir_mfma_loop_kernel(const SepArgs a, int ntiles)
     // The six-output strip code for float input takes its lane index afresh
     // in each tile: left to itself the compiler computes the lane-derived
     // offsets once, before the loop, and holds them through it (3840 x 2160
-    // six outputs 1 % faster).  The one-output loop ran 2.5-6 % slower so,
-    // and u8 input at radius class 8 3.5 % slower (its registers then fit
-    // three waves per SIMD, and the grid, the resident workgroups, grew by
-    // half): they keep the hoisted offsets.
-    constexpr bool FRESH = MODE == MODE_GAUSS || sizeof(IN) < 4;
+    // six outputs 1 % faster).  The one-output loop does so for 16-bit input at
+    // radius class 16 alone (4096 x 4096 bf16 29.4 against 31.4 us): u8 runs 3-7
+    // % slower so, bf16 at radius class 8 6 % (23.0 against 21.6 us).
+    constexpr bool FRESH = MODE == MODE_GAUSS || (sizeof(IN) == 2 && RC == 16);
+    // The next window goes into LDS before the tile's first stores, so that the
+    // wait for its loads is not one for the stores too; or, one output of 16-bit
+    // input at radius class 8, behind them: that tile's work is too short to
+    // cover the loads (4096 x 4096 bf16 23.0 -> 21.5 us).
+    constexpr bool LATE = MODE == MODE_TAPS && sizeof(IN) == 2 && RC == 8;
     // Output rows that do not start at 128-byte lines: the tiles row by row, so
     // that tiles which meet in a line run at about the same time and L2 merges
     // their parts of it (3001 x 4003 packed, radius 16: bf16 66 -> 58 us, f32 91
@@ -1364,9 +1391,12 @@ sepfir_mfma_loop_kernel(const SepArgs a, int ntiles)
                 pos = place(t);
                 mwin_load<RC, WY, MWAVES / WY, IN>(a, tid, pos.ty, pos.tx, v);
             }
-            const auto next = [&] { if (more) mwin_store<RC, WY, MWAVES / WY, IN>(tid, win, v); };
-            if (now.live) mfma_filter<RC, IN, OUT, MODE, CPOL_NT, FRESH>(a, now.y0, now.x0, p, T, stage, next);
-            else          next();
+            const auto next = [&](bool here) { if (more && here) mwin_store<RC, WY, MWAVES / WY, IN>(tid, win, v); };
+            if (now.live)
+                mfma_filter<RC, IN, OUT, MODE, CPOL_NT, FRESH>(a, now.y0, now.x0, p, T, stage, [&] { next(!LATE); });
+            else
+                next(!LATE);
+            next(LATE);
             if (!more) break;
         }
     } else {
@@ -1388,17 +1418,34 @@ sepfir_mfma_loop_kernel(const SepArgs a, int ntiles)
     }
 }
 
+inline int mfma_cus()
+{
+    int dev = 0, ncu = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+    return std::max(1, ncu);
+}
+
 // Workgroups resident at once on the whole GPU for this instantiation.
 template <class K>
 int mfma_resident(K kernel)
 {
-    int dev = 0, ncu = 0, per_cu = 0;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+    int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), 64 * MWAVES, 0)
             != hipSuccess || per_cu < 1)
         per_cu = 1;
-    return std::max(1, ncu) * per_cu;
+    return mfma_cus() * per_cu;
+}
+
+// Workgroups of a tile loop over n tiles, at most resident of them: the
+// fewest per CU that take no more rounds (4096 x 4096 u8 one output, 16 tiles
+// a CU: 17.2 us with five workgroups per CU, 16.6 with four).
+inline int mfma_loop_grid(int n, int resident)
+{
+    static const int ncu = mfma_cus();
+    const int64_t rounds = (int64_t(n) + resident - 1) / resident;
+    const int64_t per_cu = (n + rounds * ncu - 1) / (rounds * ncu);
+    return int(std::min<int64_t>({int64_t(n), int64_t(resident), per_cu * ncu}));
 }
 
 // One image in the region of a: one workgroup per WYR-shaped tile where they
@@ -1418,7 +1465,7 @@ hipError_t launch_sepfir_mfma(const SepArgs& a, int nblocks, hipStream_t s)
     if (n <= one)
         hipLaunchKernelGGL((sepfir_mfma_kernel<RC, WYR, IN, OUT, MODE>), dim3(int(n)), dim3(64 * MWAVES), 0, s, r);
     else
-        hipLaunchKernelGGL((sepfir_mfma_loop_kernel<RC, WYL, IN, OUT, MODE>), dim3(std::min(nblocks, loop)),
+        hipLaunchKernelGGL((sepfir_mfma_loop_kernel<RC, WYL, IN, OUT, MODE>), dim3(mfma_loop_grid(nblocks, loop)),
                            dim3(64 * MWAVES), 0, s, a, nblocks);
     return hipGetLastError();
 }
