@@ -872,7 +872,9 @@ __device__ __forceinline__ void mfma_ops_win(const A& a, const char* win, int la
         float mx = 0.f;
         if constexpr (std::is_same_v<IN, bf16_t>) {
             // the upper value of a pair with the lower one's bits below its
-            // own: they change neither its exponent nor what is not finite
+            // own: they change neither its exponent nor what is not finite,
+            // except that of an upper 0 they leave a denormal below bfloat16's
+            // smallest (of 0 and -0.0: 2^-134), taken for 0 below
 #pragma unroll
             for (int b = 0; b < NVB; ++b)
 #pragma unroll
@@ -891,7 +893,9 @@ __device__ __forceinline__ void mfma_ops_win(const A& a, const char* win, int la
                 }
             mx = __builtin_elementwise_maximum(float(m2[0]), float(m2[1]));
         }
-        const int ex = mfma_scale_exp(wave_max(mx), p.redo);
+        mx = wave_max(mx);
+        if constexpr (std::is_same_v<IN, bf16_t>) mx = mx < 0x1p-133f ? 0.f : mx;
+        const int ex = mfma_scale_exp(mx, p.redo);
         const float s = ldexpf(a.mq, ex);
         p.inv_s = ldexpf(1.f, -ex);
         float zero = 0.f;                       // opaque: x s + 0 stays one mixed-precision FMA
