@@ -69,9 +69,12 @@ template <int K> __device__ __forceinline__ void fma_const(float& acc, float e)
 // 16 o + 4 g + i of the accumulators gH, gV), zero outside each gradient's
 // valid region.  The vector units bound the pass (2160p u8: 8.3 M pixels), so
 // the pixel loop has no more than the sums need: the powers of a pixel's column
-// are those of w = 16 o + i - 25.5, constants, relative to the lane's column uc,
-// and u^n = (uc + sc w)^n is expanded once per strip; and only strips that
-// meet the border of the valid region mask their pixels.
+// are those of w = (16 o + i) / 64, constants, relative to the lane's first
+// column uc, and u^n = (uc + 64 sc w)^n is expanded once per strip; and only
+// strips that meet the border of the valid region mask their pixels.  uc and w
+// are not negative (the tiles start at column min(r0, r1) or later), so nothing
+// cancels in a sum of e^2 u^n; w's powers are exact in FP32 and at most 1, so
+// that no sum leaves the range of the terms it is made of.
 template <int D>
 __device__ __forceinline__ void icia_lane_moments(const SepArgs& a, int y0, int x0, v4f32* gH, v4f32* gV, float* mom,
                                                   int ms)
@@ -100,7 +103,7 @@ __device__ __forceinline__ void icia_lane_moments(const SepArgs& a, int y0, int 
         for (int n = 0; n < NU; ++n) W[xy][n] = 0.f;
     static_for<0, 4 * MNB>([&](auto pc) {
         constexpr int o = pc / 4, i = pc % 4;
-        constexpr float w = 16 * o + i - 25.5f;
+        constexpr float w = (16 * o + i) / 64.f;
         const float eH = gH[o][i], eV = gV[o][i];
         const float ee[3] = {eH * eH, eH * eV, eV * eV};
 #pragma unroll
@@ -108,19 +111,19 @@ __device__ __forceinline__ void icia_lane_moments(const SepArgs& a, int y0, int 
             W[xy][0] += ee[xy];
             static_for<1, NU>([&](auto nc) {
                 constexpr int n = nc;
-                fma_const<__builtin_bit_cast(int, icia_pow(w, n))>(W[xy][n], ee[xy]);
+                if constexpr (w != 0.f) fma_const<__builtin_bit_cast(int, icia_pow(w, n))>(W[xy][n], ee[xy]);
             });
         }
     });
-    // A[xy][n] = sum of e_X e_Y (uc + sc w)^n
+    // A[xy][n] = sum of e_X e_Y (uc + 64 sc w)^n
     float A[3][NU], up[NU], sp[NU];
     up[0] = sp[0] = 1.f;
-    up[1] = sc * (float(x0 + 4 * g) + 25.5f);
-    sp[1] = sc;
+    up[1] = sc * float(x0 + 4 * g);
+    sp[1] = 64.f * sc;
 #pragma unroll
     for (int n = 2; n < NU; ++n) {
         up[n] = up[n - 1] * up[1];
-        sp[n] = sp[n - 1] * sc;
+        sp[n] = sp[n - 1] * sp[1];
     }
 #pragma unroll
     for (int xy = 0; xy < 3; ++xy) {
