@@ -299,12 +299,14 @@ __global__ void __launch_bounds__(64) icia_reduce_kernel(const double* __restric
     if (lane == 0) moment[blockIdx.x] = float(s);
 }
 
-// Workgroups of one ICIA launch over ntiles tiles: the resident workgroups,
-// or more so that none takes more than ICIA_MAX_TILES tiles.
-template <class K>
-int icia_grid(K kernel, int ntiles)
+// Workgroups of one ICIA launch over ntiles tiles: the resident workgroups of
+// its kernel (a template argument by value: every moment kernel has the same
+// function type, and each its own residency), or more so that none takes more
+// than ICIA_MAX_TILES tiles.
+template <auto KERNEL>
+int icia_grid(int ntiles)
 {
-    static const int resident = mfma_resident(kernel);
+    static const int resident = mfma_resident(KERNEL);
     const int cap = int((int64_t(ntiles) + ICIA_MAX_TILES - 1) / ICIA_MAX_TILES);
     return std::min(ntiles, std::max(resident, cap));
 }
@@ -315,7 +317,7 @@ hipError_t launch_icia(const SepArgs& a, int ntiles, double* partial, float* mom
 {
     int grid = 0;
     if (ntiles > 0) {
-        grid = icia_grid(icia_mfma_kernel<RC, IN, D>, ntiles);
+        grid = icia_grid<icia_mfma_kernel<RC, IN, D>>(ntiles);
         hipLaunchKernelGGL((icia_mfma_kernel<RC, IN, D>), dim3(grid), dim3(64 * MWAVES), 0, s, a, ntiles, partial);
     }
     hipLaunchKernelGGL(icia_reduce_kernel<icia_nm<D>()>, dim3(icia_nm<D>()), dim3(64), 0, s, partial, grid, moment);
