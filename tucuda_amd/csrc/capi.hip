@@ -101,6 +101,15 @@ bool fir_use_mfma()
 int launch(const KernelEntry& k, SepArgs& a, hipStream_t s);
 const void* mfma_tabs_for(const SepArgs& a, int mode, hipStream_t s);
 
+// The largest input magnitude that strips take to the matrix products
+// (SepArgs::xmax): any finite one, or none where a lobe (its sum of magnitudes
+// l1, its scale mp) is not in float's range.
+constexpr float XMAX_ANY = 3.4e38f, XMAX_NONE = -1.f;
+float lobe_xmax(float l1, float mp)
+{
+    return l1 <= XMAX_ANY && mp <= XMAX_ANY ? XMAX_ANY : XMAX_NONE;     // false for a NaN
+}
+
 // One-output matrix-core launch: full taps vt / ht (tap o at index o + 16)
 // go to a.tv / a.th with their power-of-two scales (mfma.h, MODE_TAPS).
 int launch_fir_mfma(SepArgs& a, const float* vt, const float* ht, int rV, int rH, int in_dt, int out_dt,
@@ -109,6 +118,7 @@ int launch_fir_mfma(SepArgs& a, const float* vt, const float* ht, int rV, int rH
     std::memcpy(a.tv, vt, sizeof(a.tv));
     std::memcpy(a.th, ht, sizeof(a.th));
     int e[2] = {0, 0}, eq = 0;
+    a.xmax = XMAX_ANY;
     for (int l = 0; l < 2; ++l) {
         const float* t = l == 0 ? vt : ht;
         float cmax = 0.f, l1 = 0.f;
@@ -117,6 +127,7 @@ int launch_fir_mfma(SepArgs& a, const float* vt, const float* ht, int rV, int rH
         (void)std::frexp(cmax, &x);             // cmax < 2^x
         e[l] = MFMA_TAP_EXP - x;
         a.mp[l] = std::ldexp(1.f, e[l]);
+        a.xmax = std::min(a.xmax, lobe_xmax(l1, a.mp[l]));
         if (l == 0) (void)std::frexp(l1 * a.mp[0], &eq);   // l1 * mp < 2^eq
     }
     eq = std::max(eq, 0);
@@ -179,11 +190,12 @@ void centre_index(const float* lobe, int r, bool symmetric, float c[KMAX])
 // lobe l times mp[l] peak in [2^5, 2^6); mq makes mq * mp[l] * (L1 norm of
 // lobe l) <= 1 for every lobe, so that fields of an input scaled below 2^13
 // stay below 2^13; mu[k] undoes the tap and input scales of output k = (H
-// lobe, V lobe).
-void mfma_scales(SepArgs& a)
+// lobe, V lobe).  Lobes that no output of `live` uses do not decide xmax.
+void mfma_scales(SepArgs& a, unsigned live)
 {
     static const int HV[6][2] = {{0, 0}, {1, 0}, {0, 1}, {2, 0}, {1, 1}, {0, 2}};
     int ep[3], emax = 0;
+    a.xmax = XMAX_ANY;
     for (int l = 0; l < 3; ++l) {
         float cmax = 0.f, l1 = 0.f;
         for (int k = 0; k < KMAX; ++k) {
@@ -195,6 +207,8 @@ void mfma_scales(SepArgs& a)
         (void)std::frexp(cmax, &e);             // cmax < 2^e
         ep[l] = MFMA_TAP_EXP - e;
         a.mp[l] = std::ldexp(1.f, ep[l]);
+        for (int k = 0; k < 6; ++k)
+            if ((live >> k & 1u) && (HV[k][0] == l || HV[k][1] == l)) a.xmax = std::min(a.xmax, lobe_xmax(l1, a.mp[l]));
         (void)std::frexp(l1 * a.mp[l], &e);     // l1 * mp < 2^e
         emax = std::max(emax, e);
     }
@@ -540,7 +554,7 @@ int gauss_args(const float* const lobes[3], const int n[3], const tucu_image* in
         if ((rc = set_out(a, k, outs[k], rvk[k], rhk[k], shift != 0))) return rc;
     }
     if ((rc = finish_args(a, *in, live, outs, rvk, rhk))) return rc;
-    mfma_scales(a);
+    mfma_scales(a, live);
     a.mask = live;
     a.rt = GAUSS_RADII[gauss_class(rmax)];
     return TUCU_OK;
@@ -937,7 +951,7 @@ int tucu_icia_moment(const float* lobe0, int n0, const float* lobe1, int n1, con
         a.r[0] = r0; a.r[1] = r1;
         centre_index(lobe0, r0, true, a.cv[0]);
         centre_index(lobe1, r1, false, a.cv[1]);
-        mfma_scales(a);
+        mfma_scales(a, live);
         a.mask = live;
         a.rt = std::max(r0, r1) <= 8 ? 8 : 16;
         a.tabs = mfma_tabs_for(a, MODE_GAUSS, static_cast<hipStream_t>(stream));

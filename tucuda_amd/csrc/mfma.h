@@ -37,7 +37,8 @@
 // halves subnormal below half the strip's largest value: 20x the error on
 // an image whose strips mix 0..255 data with values of 10^6).
 // A strip whose input holds a NaN or an Inf, or whose largest magnitude the
-// scale cannot bring into range, is filtered by the FP32 form
+// scale cannot bring into range, is filtered by the FP32 form, and so is every
+// strip where a tap is not finite or a lobe so small that its scale overflows
 // (mfma_strip_fp32), which reaches exactly the outputs whose window holds
 // a non-finite input, as the reference's tap sums do.
 #pragma once
@@ -750,13 +751,14 @@ __device__ __forceinline__ void mfma_load(const A& a, int y0, int x0, MfmaRaw& r
 // mx: the exponent ex puts it in [2^12, 2^13).  Strips whose largest magnitude
 // is below 2^-87 or above 2^113 are out of the scale's reach (their scaled
 // values would lose precision or overflow f16), and strips with a NaN or an
-// Inf (mx is then one) would spread it: the FP32 form filters them.
-__device__ __forceinline__ int mfma_scale_exp(float mx, bool& redo)
+// Inf (mx is then one) would spread it: the FP32 form filters them, and every
+// strip of a launch whose taps have no scale (xmax).
+__device__ __forceinline__ int mfma_scale_exp(float mx, float xmax, bool& redo)
 {
     int ex;
     (void)frexpf(mx, &ex);                      // mx < 2^ex
     ex = 13 - ex;
-    redo = ex < -100 || ex > 100 || !(mx <= 3.4e38f);
+    redo = ex < -100 || ex > 100 || !(mx <= xmax);
     return ex;
 }
 
@@ -770,7 +772,7 @@ __device__ __forceinline__ void mfma_ops_raw(const A& a, const MfmaRaw& raw, Mfm
     for (int b = 0; b < G::NVB; ++b)
 #pragma unroll
         for (int j = 0; j < G::NLD; ++j) mx = __builtin_elementwise_maximum(mx, fabsf(raw[b][j]));   // keeps a NaN
-    const int ex = mfma_scale_exp(wave_max(mx), p.redo);
+    const int ex = mfma_scale_exp(wave_max(mx), a.xmax, p.redo);
     const float s = ldexpf(a.mq, ex);
     p.inv_s = ldexpf(1.f, -ex);
 #pragma unroll
@@ -895,7 +897,7 @@ __device__ __forceinline__ void mfma_ops_win(const A& a, const char* win, int la
         }
         mx = wave_max(mx);
         if constexpr (std::is_same_v<IN, bf16_t>) mx = mx < 0x1p-133f ? 0.f : mx;
-        const int ex = mfma_scale_exp(mx, p.redo);
+        const int ex = mfma_scale_exp(mx, a.xmax, p.redo);
         const float s = ldexpf(a.mq, ex);
         p.inv_s = ldexpf(1.f, -ex);
         float zero = 0.f;                       // opaque: x s + 0 stays one mixed-precision FMA

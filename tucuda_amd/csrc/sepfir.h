@@ -84,6 +84,8 @@ struct SepArgs {
     int      rt;                   // template radius class the tile grid was laid out for (batches)
     float    mp[3], mq;            // matrix-core kernels: power-of-two scales of each lobe's taps
     float    mu[6];                // and of the input, and the factor that undoes them per output
+    float    xmax;                 // largest input magnitude for which a strip takes the products; below 0
+                                   // (no strip does) if a lobe's taps or scale are out of range
     uintptr_t obase[6];            // output k: address of the element for centre (0, 0), i.e.
                                    // data + (dy_k * stride + dx_k) * elem (may lie before data)
     int32_t  ostride[6];           // output row stride, elements
