@@ -293,11 +293,11 @@ template <int ES, int S, int CPOL>
 __device__ __forceinline__ void store_piece(__amdgpu_buffer_rsrc_t r, const char* p, int at)
 {
     if constexpr (S * ES == 8)
-        __builtin_amdgcn_raw_buffer_store_b64(*reinterpret_cast<const v2u32*>(p), r, at, 0, CPOL);
+        __builtin_amdgcn_raw_buffer_store_b64(*reinterpret_cast<const v2u32_any*>(p), r, at, 0, CPOL);
     else if constexpr (S * ES == 4)
-        __builtin_amdgcn_raw_buffer_store_b32(*reinterpret_cast<const uint32_t*>(p), r, at, 0, CPOL);
+        __builtin_amdgcn_raw_buffer_store_b32(*reinterpret_cast<const u32_any*>(p), r, at, 0, CPOL);
     else if constexpr (S * ES == 2)
-        __builtin_amdgcn_raw_buffer_store_b16(*reinterpret_cast<const uint16_t*>(p), r, at, 0, CPOL);
+        __builtin_amdgcn_raw_buffer_store_b16(*reinterpret_cast<const u16_any*>(p), r, at, 0, CPOL);
     else
         __builtin_amdgcn_raw_buffer_store_b8(*reinterpret_cast<const uint8_t*>(p), r, at, 0, CPOL);
 }
@@ -338,7 +338,7 @@ store_rows(__amdgpu_buffer_rsrc_t r, uintptr_t base, const char* src, int r0, in
         const uint32_t seg = uint32_t(base) + uint32_t(at);                     // low bits of the row's address
         const int f0 = int(-seg & 127u), f1 = 256 - int((seg + 256) & 127u);    // the whole lines of the row
         const bool whole = c >= f0 && c + 16 <= f1;
-        const v4u32 q = *reinterpret_cast<const v4u32*>(src + 4 * i * PITCH);
+        const v4u32 q = *reinterpret_cast<const v4u32_any*>(src + 4 * i * PITCH);
         __builtin_amdgcn_raw_buffer_store_b128(q, r, whole ? at + c : MINVALID, 0, CPOL_NT);
         __builtin_amdgcn_raw_buffer_store_b128(q, r, whole ? MINVALID : at + c, 0, 0);
     }
@@ -1082,6 +1082,7 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& 
             Px<OUT>::pack4(sb + m * ST::PITCH + (16 * o + 4 * g) * ST::ES, r[0], r[1], r[2], r[3]);
         }
         if (k == (l == 0 ? 0 : l == 1 ? 2 : 5)) hook();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
         __builtin_amdgcn_wave_barrier();
         const int r0 = lane / ST::LPR, c0 = lane % ST::LPR * ST::EPL;
         const char* const src = sb + r0 * ST::PITCH + c0 * ST::ES;
@@ -1119,7 +1120,7 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& 
 #pragma unroll
                 for (int i = 0; i < ST::NI; ++i)
                     __builtin_amdgcn_raw_buffer_store_b128(
-                        *reinterpret_cast<const v4u32*>(src + i * ST::RPI * ST::PITCH), orsrc,
+                        *reinterpret_cast<const v4u32_any*>(src + i * ST::RPI * ST::PITCH), orsrc,
                         in && (rows >> i & 1u) ? off + i * ST::RPI * pitch : MINVALID, 0, CP);
             };
             const auto streaming = std::integral_constant<int, CPOL>{};
@@ -1165,10 +1166,11 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& 
             for (int i = 0; i < ST::NI; ++i) {
                 const int row = i * ST::RPI + r0, y = y0 + row;
                 if (y < rv || y >= a.nrow - rv) continue;
-                const v4u32 q = *reinterpret_cast<const v4u32*>(src + i * ST::RPI * ST::PITCH);
+                const v4u32 q = *reinterpret_cast<const v4u32_any*>(src + i * ST::RPI * ST::PITCH);
                 store_chunk<ST::ES>(base + uintptr_t(row * pitch64 + c0 * ST::ES), q, xa, xb);
             }
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
         __builtin_amdgcn_wave_barrier();
 #ifdef TUCU_TIMELINE
         if constexpr (CPOL == CPOL_NT_WT && MODE == MODE_GAUSS && RC == 16 && std::is_same_v<IN, float> &&

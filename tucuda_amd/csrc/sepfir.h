@@ -113,6 +113,13 @@ constexpr int CPOL_NT_WT = 2 | 16;
 
 typedef uint32_t v4u32 __attribute__((ext_vector_type(4)));
 
+// Words of a staging area in LDS, written in one width and read in another:
+// types that may alias any.
+typedef uint16_t u16_any __attribute__((may_alias));
+typedef uint32_t u32_any __attribute__((may_alias));
+typedef v2u32    v2u32_any __attribute__((may_alias));
+typedef v4u32    v4u32_any __attribute__((may_alias));
+
 // ----------------------------------------------------------------- pixels
 template <class T> struct Px;
 
@@ -133,7 +140,7 @@ template <> struct Px<float> {
     // four adjacent pixels into LDS
     static __device__ __forceinline__ void pack4(char* p, float a, float b, float c, float d)
     {
-        *reinterpret_cast<v4f32*>(p) = v4f32{a, b, c, d};
+        *reinterpret_cast<v4u32_any*>(p) = __builtin_bit_cast(v4u32, v4f32{a, b, c, d});
     }
 };
 
@@ -159,7 +166,7 @@ template <> struct Px<uint8_t> {
     // four adjacent pixels into LDS
     static __device__ __forceinline__ void pack4(char* p, float a, float b, float c, float d)
     {
-        *reinterpret_cast<uint32_t*>(p) = cvt(a) | cvt(b) << 8 | cvt(c) << 16 | cvt(d) << 24;
+        *reinterpret_cast<u32_any*>(p) = cvt(a) | cvt(b) << 8 | cvt(c) << 16 | cvt(d) << 24;
     }
 };
 
@@ -180,7 +187,7 @@ template <> struct Px<f16_t> {
     // four adjacent pixels into LDS
     static __device__ __forceinline__ void pack4(char* p, float a, float b, float c, float d)
     {
-        *reinterpret_cast<v2u32*>(p) = v2u32{pack_f16(a, b), pack_f16(c, d)};
+        *reinterpret_cast<v2u32_any*>(p) = v2u32{pack_f16(a, b), pack_f16(c, d)};
     }
 };
 
@@ -204,7 +211,7 @@ template <> struct Px<bf16_t> {
     // four adjacent pixels into LDS
     static __device__ __forceinline__ void pack4(char* p, float a, float b, float c, float d)
     {
-        *reinterpret_cast<v2u32*>(p) = v2u32{pack_bf16(a, b), pack_bf16(c, d)};
+        *reinterpret_cast<v2u32_any*>(p) = v2u32{pack_bf16(a, b), pack_bf16(c, d)};
     }
 };
 
