@@ -273,18 +273,24 @@ template <class OUT> struct MStage {
 
 typedef v4u32 v4u32u __attribute__((aligned(1)));
 
-// Stores the elements [xa, xb) (of 16 / ES, ES bytes each) of q at p.
-template <int ES> __device__ __forceinline__ void store_chunk(uintptr_t p, v4u32 q, int xa, int xb)
+// Stores the elements [xa, xb) (of 16 / ES, ES bytes each) of the chunk at q in
+// LDS at p.  Rarely taken in part, so by a loop: unrolled for the six outputs of
+// a u8 -> u8 launch it spilled 143 scalar registers of the radius-8 tile loop
+// (48 so).
+template <int ES> __device__ __forceinline__ void store_chunk(uintptr_t p, const char* q, int xa, int xb)
 {
     constexpr int E = 16 / ES;
     using T = std::conditional_t<ES == 4, uint32_t, std::conditional_t<ES == 2, uint16_t, uint8_t>>;
     if (xa <= 0 && xb >= E) {
-        *reinterpret_cast<gptr<v4u32u>>(p) = q;
+        *reinterpret_cast<gptr<v4u32u>>(p) = *reinterpret_cast<const v4u32_any*>(q);
         return;
     }
-#pragma unroll
-    for (int e = 0; e < E; ++e)
-        if (e >= xa && e < xb) reinterpret_cast<gptr<T>>(p)[e] = T(q[e * ES / 4] >> (8 * (e * ES % 4)));
+#pragma unroll 1
+    for (int e = max(xa, 0); e < min(xb, E); ++e) {
+        if constexpr (ES == 4)      reinterpret_cast<gptr<T>>(p)[e] = reinterpret_cast<const u32_any*>(q)[e];
+        else if constexpr (ES == 2) reinterpret_cast<gptr<T>>(p)[e] = reinterpret_cast<const u16_any*>(q)[e];
+        else                        reinterpret_cast<gptr<T>>(p)[e] = reinterpret_cast<const uint8_t*>(q)[e];
+    }
 }
 
 // Stores S elements (of ES bytes) from LDS through a buffer, at offset at
@@ -1109,7 +1115,12 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& 
         const uintptr_t base = a.obase[k] + uintptr_t(y0 * pitch64 + int64_t(x0) * ST::ES);
         const int rv = a.r[v], rh = a.r[h];
         const int x = x0 + c0, xa = rh - x, xb = a.ncol - rh - x;          // valid pixels of the chunk: [xa, xb)
-        if ((ST::ES == 4 || a.aligned) && !a.far) {
+        // An image hardly wider than its border may cut a chunk at both ends: the
+        // plain form below.  (A loop over such a chunk's pixels here cost the u8
+        // -> u8 launches 66 spilled vector registers: 3840 x 2160 radius 16 42
+        // us, 27 without it.)
+        const bool narrow = a.ncol - 2 * rh < ST::EPL;
+        if ((ST::ES == 4 || a.aligned) && !a.far && !narrow) {
             const __amdgpu_buffer_rsrc_t orsrc =
                 __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base), short(0), 0x7fffffff, BUF_DWORD3);
             const int off = r0 * pitch + c0 * ST::ES;
@@ -1138,36 +1149,23 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& 
                     const int y = y0 + i * ST::RPI + r0;
                     rows |= unsigned(y >= rv && y < a.nrow - rv) << i;
                 }
-                const bool cut = !in && hi > lo, both = lo > 0 && hi < ST::EPL;
+                const bool cut = !in && hi > lo;
                 const bool cuts = __builtin_amdgcn_ballot_w64(cut) != 0;
                 // a cut line is written by two instructions: ordinary stores, which merge
                 if (a.lines && !cuts) chunks(streaming, in, rows);
                 else                  chunks(ordinary, in, rows);
-                // cut at one end; a chunk cut at both (an image hardly wider
-                // than its border) pixel by pixel
                 if (cuts)
                     store_cut<ST::ES, 0, ST::NI>(orsrc, src, ST::RPI * ST::PITCH, off, ST::RPI * pitch, lo > 0,
-                                                 cut && !both ? hi - lo : 0, rows);
-                if (__builtin_amdgcn_ballot_w64(cut && both)) {
-#pragma unroll 1
-                    for (int e = 0; e < ST::EPL; ++e)
-#pragma unroll
-                        for (int i = 0; i < ST::NI; ++i)
-                            store_piece<ST::ES, 1, 0>(
-                                orsrc, src + e * ST::ES + i * ST::RPI * ST::PITCH,
-                                cut && both && e >= lo && e < hi && (rows >> i & 1u)
-                                    ? off + e * ST::ES + i * ST::RPI * pitch : MINVALID);
-                }
+                                                 cut ? hi - lo : 0, rows);
             }
         } else {
             // 16-bit and 8-bit rows that are not aligned to four pixels, rows
-            // too far apart: plain addresses, ordinary stores
+            // too far apart, narrow images: plain addresses, ordinary stores
 #pragma unroll
             for (int i = 0; i < ST::NI; ++i) {
                 const int row = i * ST::RPI + r0, y = y0 + row;
                 if (y < rv || y >= a.nrow - rv) continue;
-                const v4u32 q = *reinterpret_cast<const v4u32_any*>(src + i * ST::RPI * ST::PITCH);
-                store_chunk<ST::ES>(base + uintptr_t(row * pitch64 + c0 * ST::ES), q, xa, xb);
+                store_chunk<ST::ES>(base + uintptr_t(row * pitch64 + c0 * ST::ES), src + i * ST::RPI * ST::PITCH, xa, xb);
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
