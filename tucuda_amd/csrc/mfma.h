@@ -1099,13 +1099,17 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& 
         // overwrite the data, and some lanes then stored the new value.
         // At the edge of the valid region a lane whose pixels all lie outside
         // takes an offset past the buffer, which drops its store, and the few
-        // chunks an edge cuts store in pieces.  Edge strips keep the policy of
-        // the others where no chunk is cut: lines left dirty in L2 by ordinary
-        // stores are written back when the kernel ends (3840 x 2160 f32 six
-        // outputs: 54.7 us with ordinary stores in the edge strips, 49.6 so).
-        // With a chunk cut (radii that are not a multiple of the chunk), the
-        // streaming pieces of a line cost more than that (256 images of mixed
-        // radii, f32: 1.30 against 1.20 ms).
+        // chunks an edge cuts store in pieces.  Where the edge lies within a
+        // line, the strip writes a part of it: streamed, that part goes to
+        // memory by itself, stored ordinarily it stays in L2 until the kernel
+        // ends.  Float strips stream it only from WHOLE bytes of a line up:
+        // whole lines in the tile loops, halves in a one-round launch (six
+        // outputs f32, streaming against ordinary: 1080p radius 4, 16 bytes cut,
+        // 14.4 against 12.6 us, radius 16, half a line, 14.1 against 14.8; 3840
+        // x 2160 radius 4 47.5 against 43.3, radius 16 50.0 against 49.0).
+        // 16-bit strips stream it wherever no chunk is cut (1080p bf16 radius
+        // 16, a quarter line, 11.1 us, ordinary 11.9).  A chunk that is cut
+        // stores in two instructions, which only L2 merges: ordinary.
         // Rows that do not start at 128-byte lines take ordinary stores where
         // strips meet in a line (store_rows) or, where no line lies within a
         // strip's row or in a one-round launch, throughout (one-round 1080 x
@@ -1151,9 +1155,11 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& 
                 }
                 const bool cut = !in && hi > lo;
                 const bool cuts = __builtin_amdgcn_ballot_w64(cut) != 0;
-                // a cut line is written by two instructions: ordinary stores, which merge
-                if (a.lines && !cuts) chunks(streaming, in, rows);
-                else                  chunks(ordinary, in, rows);
+                // the valid bytes of the strip's row: [e0, e1)
+                const int e0 = max(rh - x0, 0) * ST::ES, e1 = min(a.ncol - rh - x0, MSTRIP_W) * ST::ES;
+                constexpr int WHOLE = ST::ES < 4 ? 16 : CPOL == CPOL_NT ? 128 : 64;
+                if (a.lines && ((e0 | e1) & (WHOLE - 1)) == 0) chunks(streaming, in, rows);
+                else                                           chunks(ordinary, in, rows);
                 if (cuts)
                     store_cut<ST::ES, 0, ST::NI>(orsrc, src, ST::RPI * ST::PITCH, off, ST::RPI * pitch, lo > 0,
                                                  cut ? hi - lo : 0, rows);
