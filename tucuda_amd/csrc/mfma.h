@@ -384,6 +384,36 @@ mfma_load_block(const A& a, __amdgpu_buffer_rsrc_t rsrc, int y0, int x0, int b, 
     }
 }
 
+// The same for 16-bit input, in 32-bit registers as stored, of one-output
+// strips of radius class 8 (see MFMA_DIRECT).  Windows inside the image load
+// at uniform row bases plus a 32-bit lane offset: the zero-extending form, so
+// that no mask right after the loads makes the wave wait for them.  At the
+// image's edge the same loads at clamped addresses, and 0 outside.
+template <bool INSIDE, class A>
+__device__ __forceinline__ void mfma_load_block16(const A& a, int y0, int x0, int b, int g, int m, uint32_t* v)
+{
+    constexpr int RC = 8;
+    const int col = x0 - RC + 16 * b + m, sb = a.in_stride_b;
+    const char* const in = static_cast<const char*>(a.in);
+    const auto ld = [](const char* row, uint32_t off) -> uint32_t {
+        return *reinterpret_cast<gptr<const uint16_t>>(reinterpret_cast<uintptr_t>(row) + off);
+    };
+    if constexpr (INSIDE) {
+        const uint32_t off = uint32_t(8 * g * sb + 2 * col);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = ld(in + int64_t(y0 - RC + j) * sb, off);
+    } else {
+        const bool colok = unsigned(col) < unsigned(a.ncol);
+        const uint32_t off = uint32_t(2 * min(max(col, 0), a.ncol - 1));
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int row = y0 - RC + 8 * g + j;
+            const uint32_t x = ld(in + int64_t(min(max(row, 0), a.nrow - 1)) * sb, off);
+            v[j] = colok && unsigned(row) < unsigned(a.nrow) ? x : 0u;
+        }
+    }
+}
+
 // ------------------------------------------------------------ input window
 // u8, f16 and bf16 input reaches the strips through LDS: the workgroup loads
 // the window of its tile (SY strips down by SX across, and the radius class
@@ -695,6 +725,7 @@ __device__ __forceinline__ ConstArgs& opaque_args(const SepArgs&)
 // (mfma_load_block's order); radius class 8 uses blocks 0 .. 4 and entries
 // 0 .. 7.
 using MfmaRaw = float[6][12];
+using MfmaRaw16 = uint32_t[MGeo<8>::NVB][8];    // of 16-bit input (mfma_load_block16)
 
 // A strip's matrix operands of the vertical pass, and its scale.
 // xh / xl: entries 0 .. 7 (rows 8 g + j), high and low halves; xt (K = 48):
@@ -723,6 +754,15 @@ constexpr int MFMA_WAVES_PER_SIMD = 3;
 // where it needs 128 registers or fewer).
 template <class IN> constexpr int MFMA_LOOP_WAVES = sizeof(IN) == 4 ? 2 : 3;
 
+// Strips of the tile loop that load their 16-bit input themselves, without the
+// window in LDS: one output of radius class 8 is too little work per tile to
+// cover the window's way through LDS and its two barriers (4096 x 4096 17 x 17
+// taps bf16 22.5 -> 18.9 us, f16 21.4 -> 18.3; 16 columns more per strip, at
+// radius class 16, are loaded faster by the workgroup: 52 us so, 30 by the
+// window; u8 halves the window's bytes).
+template <int RC, class IN, int MODE>
+constexpr bool MFMA_DIRECT = MODE == MODE_TAPS && RC == 8 && sizeof(IN) == 2;
+
 // Issues the loads of the float strip at (y0, x0); the values arrive in raw.
 // FRESH: the lane index is opaque to the compiler (a caller's loop then
 // recomputes what derives from it in each pass instead of holding it).
@@ -750,6 +790,21 @@ __device__ __forceinline__ void mfma_load(const A& a, int y0, int x0, MfmaRaw& r
     if constexpr (!G::K48) {
 #pragma unroll
         for (int b = 0; b < G::NVB; ++b) raw[b][8] = raw[b][9] = raw[b][10] = raw[b][11] = 0;
+    }
+}
+
+// The same of a 16-bit strip, radius class 8.
+template <class A> __device__ __forceinline__ void mfma_load16(const A& a, int y0, int x0, MfmaRaw16& raw)
+{
+    using G = MGeo<8>;
+    const int lane = threadIdx.x & 63, g = lane >> 4, m = lane & 15;
+    const bool inside = y0 >= 8 && y0 - 8 + G::KV <= a.nrow && x0 >= 8 && x0 - 8 + 16 * G::NVB <= a.ncol;   // uniform
+    if (inside) {
+#pragma unroll
+        for (int b = 0; b < G::NVB; ++b) mfma_load_block16<true>(a, y0, x0, b, g, m, raw[b]);
+    } else {
+#pragma unroll
+        for (int b = 0; b < G::NVB; ++b) mfma_load_block16<false>(a, y0, x0, b, g, m, raw[b]);
     }
 }
 
@@ -811,6 +866,31 @@ template <class IN> __device__ __forceinline__ v2f16 scale_pair(uint32_t w, floa
         hi = float(h[1]);
     }
     return v2f16{_Float16(__builtin_fmaf(lo, s, zero)), _Float16(__builtin_fmaf(hi, s, zero))};
+}
+
+// The operands of a 16-bit strip of radius class 8 from its loaded values.
+template <class IN, class A>
+__device__ __forceinline__ void mfma_ops_raw16(const A& a, const MfmaRaw16& raw, MfmaOps& p)
+{
+    constexpr int NVB = MGeo<8>::NVB;
+    const auto value = [](uint32_t v) -> float {
+        if constexpr (std::is_same_v<IN, f16_t>) return float(__builtin_bit_cast(_Float16, uint16_t(v)));
+        else                                     return __uint_as_float(v << 16);
+    };
+    float mx = 0.f;
+#pragma unroll
+    for (int b = 0; b < NVB; ++b)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) mx = __builtin_elementwise_maximum(mx, fabsf(value(raw[b][j])));     // keeps a NaN
+    const int ex = mfma_scale_exp(wave_max(mx), a.xmax, p.redo);
+    const float s = ldexpf(a.mq, ex);
+    p.inv_s = ldexpf(1.f, -ex);
+    float zero = 0.f;                           // opaque: x s + 0 stays one mixed-precision FMA
+    asm("" : "+v"(zero));
+#pragma unroll
+    for (int b = 0; b < NVB; ++b)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) p.xh[b][j] = _Float16(__builtin_fmaf(value(raw[b][j]), s, zero));
 }
 
 // Two u8 values (bytes I, I + 1 of w) as f16 times s, exactly: with M = 1024 s
@@ -1362,18 +1442,14 @@ sepfir_mfma_loop_kernel(const SepArgs a, int ntiles)
     int t = mfma_share_lo(ntiles, grid, x) + b / QN;
     float* const stage = reinterpret_cast<float*>(stage4) + (threadIdx.x >> 6) * 16 * MOPITCH;
     if (t >= hi) return;                            // uniform over the workgroup
-    // The six-output strip code for float input takes its lane index afresh
-    // in each tile: left to itself the compiler computes the lane-derived
+    // The six-output strip code takes its lane index afresh in each tile: left to itself the compiler computes the lane-derived
     // offsets once, before the loop, and holds them through it (3840 x 2160
-    // six outputs 1 % faster).  The one-output loop does so for 16-bit input at
-    // radius class 16 alone (4096 x 4096 bf16 29.4 against 31.4 us): u8 runs 3-7
-    // % slower so, bf16 at radius class 8 6 % (23.0 against 21.6 us).
+    // six outputs f32 1 % faster).  The one-output loop does so for 16-bit input
+    // at radius class 16 alone (4096 x 4096 bf16 29.4 against 31.4 us): u8 runs
+    // 3-7 % slower so.
     constexpr bool FRESH = MODE == MODE_GAUSS || (sizeof(IN) == 2 && RC == 16);
     // The next window goes into LDS before the tile's first stores, so that the
-    // wait for its loads is not one for the stores too; or, one output of 16-bit
-    // input at radius class 8, behind them: that tile's work is too short to
-    // cover the loads (4096 x 4096 bf16 23.0 -> 21.5 us).
-    constexpr bool LATE = MODE == MODE_TAPS && sizeof(IN) == 2 && RC == 8;
+    // wait for its loads is not one for the stores too.
     // Output rows that do not start at 128-byte lines: the tiles row by row, so
     // that tiles which meet in a line run at about the same time and L2 merges
     // their parts of it (3001 x 4003 packed, radius 16: bf16 66 -> 58 us, f32 91
@@ -1381,7 +1457,23 @@ sepfir_mfma_loop_kernel(const SepArgs a, int ntiles)
     const int nx = a.lines ? 0 : ntiles / a.tiles_y;
     const auto place = [&](int i) { return mfma_tile_pos<WY>(a, nx ? i % nx * a.tiles_y + i / nx : i); };
     TilePos pos = place(t);
-    if constexpr (sizeof(IN) < 4) {
+    if constexpr (MFMA_DIRECT<RC, IN, MODE>) {
+        MfmaRaw16 raw;
+        if (pos.live) mfma_load16(a, pos.y0, pos.x0, raw);      // in flight while the tables are built
+        mfma_get_tabs<MODE>(a, T);
+        __syncthreads();
+        while (t < hi) {                            // uniform over the workgroup
+            if (pos.live) {
+                MfmaOps p;
+                mfma_ops_raw16<IN>(a, raw, p);
+                mfma_filter<RC, IN, OUT, MODE, CPOL_NT, FRESH>(a, pos.y0, pos.x0, p, T, stage, [] {});
+            }
+            t += step;
+            if (t >= hi) break;
+            pos = place(t);
+            if (pos.live) mfma_load16(a, pos.y0, pos.x0, raw);
+        }
+    } else if constexpr (sizeof(IN) < 4) {
         using W = MWin<RC, WY, MWAVES / WY, IN>;
         __shared__ v4u32 win4[W::BYTES / 16];
         char* const win = reinterpret_cast<char*>(win4);
@@ -1403,12 +1495,11 @@ sepfir_mfma_loop_kernel(const SepArgs a, int ntiles)
                 pos = place(t);
                 mwin_load<RC, WY, MWAVES / WY, IN>(a, tid, pos.ty, pos.tx, v);
             }
-            const auto next = [&](bool here) { if (more && here) mwin_store<RC, WY, MWAVES / WY, IN>(tid, win, v); };
+            const auto next = [&] { if (more) mwin_store<RC, WY, MWAVES / WY, IN>(tid, win, v); };
             if (now.live)
-                mfma_filter<RC, IN, OUT, MODE, CPOL_NT, FRESH>(a, now.y0, now.x0, p, T, stage, [&] { next(!LATE); });
+                mfma_filter<RC, IN, OUT, MODE, CPOL_NT, FRESH>(a, now.y0, now.x0, p, T, stage, next);
             else
-                next(!LATE);
-            next(LATE);
+                next();
             if (!more) break;
         }
     } else {
