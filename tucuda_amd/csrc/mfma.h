@@ -1541,8 +1541,8 @@ int mfma_resident(K kernel)
 }
 
 // Workgroups of a tile loop over n tiles, at most resident of them: the
-// fewest per CU that take no more rounds (4096 x 4096 u8 one output, 16 tiles
-// a CU: 17.2 us with five workgroups per CU, 16.6 with four).
+// fewest per CU that take no more rounds (2560 x 1440 u8 -> f32 six outputs,
+// radius 16: 22.5 us, 24.9 with all that fit).
 inline int mfma_loop_grid(int n, int resident)
 {
     static const int ncu = mfma_cus();
@@ -1550,6 +1550,13 @@ inline int mfma_loop_grid(int n, int resident)
     const int64_t per_cu = (n + rounds * ncu - 1) / (rounds * ncu);
     return int(std::min<int64_t>({int64_t(n), int64_t(resident), per_cu * ncu}));
 }
+
+// The most workgroups per CU of a tile loop.  One output of u8 input at radius
+// class 8 has registers for four or five and is bound by memory: with three,
+// 4096 x 4096 17 x 9 taps u8 -> f16 take 14.9 us against 16.0, -> u8 15.4 against
+// 16.0, 3840 x 2160 17 x 17 -> f32 10.4 against 10.7.
+template <int RC, class IN, int MODE>
+constexpr int MFMA_LOOP_PER_CU = MODE == MODE_TAPS && RC == 8 && sizeof(IN) == 1 ? 3 : 8;
 
 // One image in the region of a: one workgroup per WYR-shaped tile where they
 // fit the resident workgroups, else the tile loop with WYL, whose tile count
@@ -1559,7 +1566,8 @@ inline int mfma_loop_grid(int n, int resident)
 template <int RC, int WYR, int WYL, class IN, class OUT, int MODE = MODE_GAUSS>
 hipError_t launch_sepfir_mfma(const SepArgs& a, int nblocks, hipStream_t s)
 {
-    static const int loop = mfma_resident(sepfir_mfma_loop_kernel<RC, WYL, IN, OUT, MODE>);
+    static const int loop = std::min(mfma_resident(sepfir_mfma_loop_kernel<RC, WYL, IN, OUT, MODE>),
+                                     mfma_cus() * MFMA_LOOP_PER_CU<RC, IN, MODE>);
     static const int one = MODE == MODE_TAPS ? mfma_resident(sepfir_mfma_kernel<RC, WYR, IN, OUT, MODE>) : loop;
     constexpr int H = 16 * WYR, W = MSTRIP_W * (MWAVES / WYR);
     SepArgs r = a;
