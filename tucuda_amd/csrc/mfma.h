@@ -750,9 +750,17 @@ constexpr int MFMA_WAVES_PER_SIMD = 3;
 // a loop needs more registers than the one-round kernels, two waves per SIMD
 // (the one-output mode needs fewer, but at three or four it spills);
 // narrow input, which holds no float values and prefetches the next window
-// in at most 20 registers, takes three at radius class 16 (four by itself
-// where it needs 128 registers or fewer).
-template <class IN> constexpr int MFMA_LOOP_WAVES = sizeof(IN) == 4 ? 2 : 3;
+// in at most 36 registers, takes three at radius class 16 (four by itself
+// where it needs 128 registers or fewer).  Six outputs u8 -> f32 at radius class
+// 8 are scheduled for two, though their 109 registers admit four: more of a
+// strip's work then overlaps (3840 x 2160 43.6 -> 42.6 us, 4032 x 3000 62.6 ->
+// 61.4, 4608 x 3456 81.3 -> 79.7).
+template <int RC, class IN, class OUT, int MODE>
+constexpr bool MFMA_LOOP_TWO = MODE == MODE_GAUSS && RC == 8 && sizeof(IN) == 1 && sizeof(OUT) == 4;
+template <int RC, class IN, class OUT, int MODE>
+constexpr int MFMA_LOOP_WAVES = sizeof(IN) == 4 || MFMA_LOOP_TWO<RC, IN, OUT, MODE> ? 2 : 3;
+template <int RC, class IN, class OUT, int MODE>
+constexpr int MFMA_LOOP_WAVES_MAX = MFMA_LOOP_TWO<RC, IN, OUT, MODE> ? 2 : 8;
 
 // Strips of the tile loop that load their 16-bit input themselves, without the
 // window in LDS: one output of radius class 8 is too little work per tile to
@@ -1430,7 +1438,7 @@ sepfir_mfma_kernel(const SepArgs a)
 // them.  (A 4096 x 4096 FIRFilter2 launch: 21.5 us against 25.5 us with one
 // workgroup per tile, which rebuilds the tables 4096 times.)
 template <int RC, int WY, class IN, class OUT, int MODE = MODE_GAUSS>
-__global__ void __launch_bounds__(64 * MWAVES) __attribute__((amdgpu_waves_per_eu(MFMA_LOOP_WAVES<IN>)))
+__global__ void __launch_bounds__(64 * MWAVES) __attribute__((amdgpu_waves_per_eu(MFMA_LOOP_WAVES<RC, IN, OUT, MODE>, MFMA_LOOP_WAVES_MAX<RC, IN, OUT, MODE>)))
 sepfir_mfma_loop_kernel(const SepArgs a, int ntiles)
 {
     __shared__ ModeTabs<MODE> T;
@@ -1542,12 +1550,19 @@ int mfma_resident(K kernel)
 
 // Workgroups of a tile loop over n tiles, at most resident of them: the
 // fewest per CU that take no more rounds (2560 x 1440 u8 -> f32 six outputs,
-// radius 16: 22.5 us, 24.9 with all that fit).
-inline int mfma_loop_grid(int n, int resident)
+// radius 16: 22.5 us, 24.9 with all that fit).  TWO: of at most three rounds,
+// two workgroups per CU where they leave no more places idle -- six outputs
+// f32 -> f32, radius class 8, which the write stream bounds whether two or three
+// are resident, so that the emptier last round shows (3840 x 2160, 2040 tiles,
+// four rounds of 512 against three of 768: 44.7 -> 43.9 us; 3000 x 1500 27.6 ->
+// 26.7; with more rounds it goes either way: 4608 x 3456 86.8 -> 84.1, 4000 x
+// 4000 86.6 -> 89.9).
+template <bool TWO> int mfma_loop_grid(int n, int resident)
 {
     static const int ncu = mfma_cus();
-    const int64_t rounds = (int64_t(n) + resident - 1) / resident;
-    const int64_t per_cu = (n + rounds * ncu - 1) / (rounds * ncu);
+    const auto rounds = [&](int64_t grid) { return (int64_t(n) + grid - 1) / grid; };
+    int64_t per_cu = (n + rounds(resident) * ncu - 1) / (rounds(resident) * ncu);
+    if (TWO && per_cu > 2 && rounds(per_cu * ncu) <= 3 && rounds(2 * ncu) * 2 <= rounds(per_cu * ncu) * per_cu) per_cu = 2;
     return int(std::min<int64_t>({int64_t(n), int64_t(resident), per_cu * ncu}));
 }
 
@@ -1570,13 +1585,14 @@ hipError_t launch_sepfir_mfma(const SepArgs& a, int nblocks, hipStream_t s)
                                      mfma_cus() * MFMA_LOOP_PER_CU<RC, IN, MODE>);
     static const int one = MODE == MODE_TAPS ? mfma_resident(sepfir_mfma_kernel<RC, WYR, IN, OUT, MODE>) : loop;
     constexpr int H = 16 * WYR, W = MSTRIP_W * (MWAVES / WYR);
+    constexpr bool TWO = MODE == MODE_GAUSS && RC == 8 && sizeof(IN) == 4 && sizeof(OUT) == 4;
     SepArgs r = a;
     r.tiles_y = (a.cy1 - a.cy0 + H - 1) / H;
     const int64_t n = int64_t((a.cx1 - a.cx0 + W - 1) / W) * r.tiles_y;
     if (n <= one)
         hipLaunchKernelGGL((sepfir_mfma_kernel<RC, WYR, IN, OUT, MODE>), dim3(int(n)), dim3(64 * MWAVES), 0, s, r);
     else
-        hipLaunchKernelGGL((sepfir_mfma_loop_kernel<RC, WYL, IN, OUT, MODE>), dim3(mfma_loop_grid(nblocks, loop)),
+        hipLaunchKernelGGL((sepfir_mfma_loop_kernel<RC, WYL, IN, OUT, MODE>), dim3(mfma_loop_grid<TWO>(nblocks, loop)),
                            dim3(64 * MWAVES), 0, s, a, nblocks);
     return hipGetLastError();
 }
