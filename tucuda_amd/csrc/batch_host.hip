@@ -35,7 +35,10 @@ const BatchEntry& batch_entry(int fam, int thi, int in_dt, int out_dt)
 
 // bf16 batches of the matrix-core kernels take 64 x 64 tiles: their window of
 // the input is the smallest per pixel and fewer of them meet an image's edge
-// (256 images of mixed sizes: 0.78 ms against 0.90 with 32 x 128).
+// (256 images of mixed sizes: 0.78 ms against 0.90 with 32 x 128).  Float input
+// has no window.  Type pairs other than f32 -> f32 and bf16 -> bf16 have the 64 x
+// 64 shape alone, for a server that asks for 64 tile rows; a batch of such a pair
+// finds no kernel at its default shape and is refused.
 int batch_default(int fam, int in_dt, int out_dt)
 {
     return fam == BATCH_MFMA && in_dt == TUCU_BF16 && out_dt == TUCU_BF16 ? 2 : BATCH_TH_DEFAULT;

@@ -6,9 +6,9 @@
 // banded matrix products, and the vector units only split, scale and store.
 //
 // Strip: one wave64 filters 16 centre rows x 64 centre columns (4 blocks of
-// 16 columns); a workgroup puts 4 waves side by side (16 x 256), so that the
-// rows it writes are long runs (the write stream dominates the traffic).  With RC the radius
-// class (8 or 16; lobes zero-padded to it) and K = 16 + 2 RC:
+// 16 columns); a workgroup holds 4 strips, one above the other or two by two
+// (MFMA_WYS), whose halo rows meet in L1 or in a window of the input in LDS.
+// With RC the radius class (8 or 16; lobes zero-padded to it) and K = 16 + 2 RC:
 //   vertical pass, per field block b (16 input columns starting at
 //   x0 - RC + 16 b) and lobe l:
 //       F^T (16 cols x 16 rows) = X^T (16 cols x K input rows) * T_l^T (K x 16)
@@ -56,9 +56,7 @@ typedef _Float16 v8f16 __attribute__((ext_vector_type(8)));
 
 constexpr int MSTRIP_W = 64;              // centre columns per strip
 constexpr int MNB      = MSTRIP_W / 16;   // output blocks per strip
-constexpr int MWAVES   = 4;               // strips (waves) per workgroup, side by side
-constexpr int MTILE_H  = 16;              // centre rows per workgroup tile
-constexpr int MTILE_W  = MSTRIP_W * MWAVES;   // centre columns per workgroup tile
+constexpr int MWAVES   = 4;               // strips (waves) per workgroup
 constexpr int MOPITCH  = MSTRIP_W + 4;    // row pitch (floats) of a wave's output staging area
 constexpr int MT4      = 112;             // tap-run table entries per lobe
 constexpr int MBASE    = 64;              // run t starts with tap t - MBASE
@@ -330,10 +328,13 @@ store_cut(__amdgpu_buffer_rsrc_t r, const char* src, int rpitch, int at, int opi
 // instruction (16 lanes of 16 bytes each), rows pitch bytes apart in the output
 // from base, PITCH in LDS from src (the lane's first chunk, c bytes into row
 // r0): the chunks of whole lines streaming, those of the lines that the strip
-// shares with its neighbours by ordinary stores, which L2 merges.  Streaming a
-// shared line writes it to memory in parts (3001 x 4004 packed f32 six outputs:
-// 142 us), an ordinary store of a whole line leaves it dirty in L2 until it is
-// evicted (100 us); so split 64 us, as rows of whole lines take.
+// shares with its neighbours by ordinary stores, which L2 merges.  Where the row
+// starts at a 16-byte boundary (3001 x 4004 packed f32 six outputs): all
+// streamed, a shared line is written to memory in parts, 142 us; all ordinary,
+// whole lines stay dirty in L2 until they are evicted, 100; so split 62, as rows
+// of whole lines take.  Elsewhere the two chunks at the ends of a whole line
+// reach into the next and go out ordinarily, so that most of that line is
+// streamed and the rest merges: 3001 x 4003 101 us ordinary, 74 so.
 template <int PITCH>
 __device__ __forceinline__ void
 store_rows(__amdgpu_buffer_rsrc_t r, uintptr_t base, const char* src, int r0, int c, int pitch)
@@ -1196,8 +1197,11 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& 
         // 14.4 against 12.6 us, radius 16, half a line, 14.1 against 14.8; 3840
         // x 2160 radius 4 47.5 against 43.3, radius 16 50.0 against 49.0).
         // 16-bit strips stream it wherever no chunk is cut (1080p bf16 radius
-        // 16, a quarter line, 11.1 us, ordinary 11.9).  A chunk that is cut
-        // stores in two instructions, which only L2 merges: ordinary.
+        // 16, a quarter line, 11.1 us, ordinary 11.9), and so do 8-bit ones,
+        // whose rows of 64 bytes are half lines throughout (u8 -> u8 1080p radius
+        // 16 9.0 us, ordinary and tile by tile along the rows 10.4; 4096 x 4096
+        // 17 x 9 taps 15.2, 18.2).  A chunk that is cut stores in two
+        // instructions, which only L2 merges: ordinary.
         // Rows that do not start at 128-byte lines take ordinary stores where
         // strips meet in a line (store_rows) or, where no line lies within a
         // strip's row or in a one-round launch, throughout (one-round 1080 x
