@@ -269,59 +269,20 @@ template <class OUT> struct MStage {
     static_assert(PITCH <= MOPITCH * 4, "staging area too narrow");
 };
 
-typedef v4u32 v4u32u __attribute__((aligned(1)));
+typedef v4u32 v4u32u __attribute__((aligned(1), may_alias));
 
 // Stores the elements [xa, xb) (of 16 / ES, ES bytes each) of the chunk at q in
-// LDS at p.  Rarely taken in part, so by a loop: unrolled for the six outputs of
-// a u8 -> u8 launch it spilled 143 scalar registers of the radius-8 tile loop
-// (48 so).
+// LDS at p, one by one (strips that hold less than a chunk).
 template <int ES> __device__ __forceinline__ void store_chunk(uintptr_t p, const char* q, int xa, int xb)
 {
     constexpr int E = 16 / ES;
     using T = std::conditional_t<ES == 4, uint32_t, std::conditional_t<ES == 2, uint16_t, uint8_t>>;
-    if (xa <= 0 && xb >= E) {
-        *reinterpret_cast<gptr<v4u32u>>(p) = *reinterpret_cast<const v4u32_any*>(q);
-        return;
-    }
 #pragma unroll 1
     for (int e = max(xa, 0); e < min(xb, E); ++e) {
         if constexpr (ES == 4)      reinterpret_cast<gptr<T>>(p)[e] = reinterpret_cast<const u32_any*>(q)[e];
         else if constexpr (ES == 2) reinterpret_cast<gptr<T>>(p)[e] = reinterpret_cast<const u16_any*>(q)[e];
         else                        reinterpret_cast<gptr<T>>(p)[e] = reinterpret_cast<const uint8_t*>(q)[e];
     }
-}
-
-// Stores S elements (of ES bytes) from LDS through a buffer, at offset at
-// (past the buffer: nothing).
-template <int ES, int S, int CPOL>
-__device__ __forceinline__ void store_piece(__amdgpu_buffer_rsrc_t r, const char* p, int at)
-{
-    if constexpr (S * ES == 8)
-        __builtin_amdgcn_raw_buffer_store_b64(*reinterpret_cast<const v2u32_any*>(p), r, at, 0, CPOL);
-    else if constexpr (S * ES == 4)
-        __builtin_amdgcn_raw_buffer_store_b32(*reinterpret_cast<const u32_any*>(p), r, at, 0, CPOL);
-    else if constexpr (S * ES == 2)
-        __builtin_amdgcn_raw_buffer_store_b16(*reinterpret_cast<const u16_any*>(p), r, at, 0, CPOL);
-    else
-        __builtin_amdgcn_raw_buffer_store_b8(*reinterpret_cast<const uint8_t*>(p), r, at, 0, CPOL);
-}
-
-// The elements left of a chunk that an edge cuts, NI row steps of it (rpitch
-// bytes apart in LDS, opitch in the output): its last n (tail) or first n
-// elements, as pieces of E / 2, E / 4, .. 1 elements, each at most once and at
-// a multiple of its size (the bits of n).  at is the chunk's offset; row step
-// i is stored if bit i of rows is set.
-template <int ES, int CPOL, int NI, int S = 8 / ES>
-__device__ __forceinline__ void
-store_cut(__amdgpu_buffer_rsrc_t r, const char* src, int rpitch, int at, int opitch, bool tail, int n, unsigned rows)
-{
-    constexpr int E = 16 / ES;
-    const int pos = n & S ? (tail ? E - (n & ~(S - 1)) : n & ~(2 * S - 1)) : 0;
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-        store_piece<ES, S, CPOL>(r, src + pos * ES + i * rpitch,
-                                 (n & S) && (rows >> i & 1u) ? at + pos * ES + i * opitch : MINVALID);
-    if constexpr (S > 1) store_cut<ES, CPOL, NI, S / 2>(r, src, rpitch, at, opitch, tail, n, rows);
 }
 
 // Stores a strip of float rows that do not start at 128-byte lines, 4 rows an
@@ -1186,85 +1147,123 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& 
         // every output within 2^31 bytes).  No scalar offset: after a 16-byte
         // store with one the compiler lets the next vector instruction
         // overwrite the data, and some lanes then stored the new value.
-        // At the edge of the valid region a lane whose pixels all lie outside
-        // takes an offset past the buffer, which drops its store, and the few
-        // chunks an edge cuts store in pieces.  Where the edge lies within a
-        // line, the strip writes a part of it: streamed, that part goes to
-        // memory by itself, stored ordinarily it stays in L2 until the kernel
-        // ends.  Float strips stream it only from WHOLE bytes of a line up:
-        // whole lines in the tile loops, halves in a one-round launch (six
-        // outputs f32, streaming against ordinary: 1080p radius 4, 16 bytes cut,
-        // 14.4 against 12.6 us, radius 16, half a line, 14.1 against 14.8; 3840
-        // x 2160 radius 4 47.5 against 43.3, radius 16 50.0 against 49.0).
-        // 16-bit strips stream it wherever no chunk is cut (1080p bf16 radius
-        // 16, a quarter line, 11.1 us, ordinary 11.9), and so do 8-bit ones,
-        // whose rows of 64 bytes are half lines throughout (u8 -> u8 1080p radius
-        // 16 9.0 us, ordinary and tile by tile along the rows 10.4; 4096 x 4096
-        // 17 x 9 taps 15.2, 18.2).  A chunk that is cut stores in two
-        // instructions, which only L2 merges: ordinary.
+        // At the edge of the valid region a lane whose chunk lies outside takes an
+        // offset past the buffer, which drops its store; where the edge lies
+        // within a chunk, moved chunks need no store of single pixels (1291 x
+        // 1192 f32 six outputs, radius 16: 15.0 us with the pieces of a cut chunk
+        // stored one by one, 13.3 so; 823 x 519 11.4 -> 9.1, bf16 9.9 -> 8.0).
+        // A tile loop takes the strips inside the valid region first, without
+        // these conditions, and for narrow input reads what the others need from
+        // the arguments there and then (held through the loop it spilled 38
+        // scalar registers: 3840 x 2160 u8 -> f32 42.4 us, 41.8 so).
+        // Where the edge lies within a line, the strip writes a part of it:
+        // streamed, that part goes to memory by itself, stored ordinarily it
+        // stays in L2 until the kernel ends.  Float strips stream whole lines in
+        // the tile loops, in a one-round launch also halves and, at radius class
+        // 16, lines that lack their last 16 bytes alone (six outputs f32,
+        // streaming against ordinary: 1080p radius 4, 16 bytes cut at the left,
+        // 14.4 against 12.6 us, and the last 16 at the right alone 13.2 against
+        // 12.3; radius 16, half a line, 14.1 against 14.8, 1292 x 1192 the last 16
+        // bytes 11.6 against 12.7; 3840 x 2160 radius 4 47.5 against 43.3, radius
+        // 16 50.0 against 49.0).  16-bit strips stream it wherever no chunk is cut
+        // (1080p bf16 radius 16, a quarter line, 11.1 us, ordinary 11.9), and so
+        // do 8-bit ones, whose rows of 64 bytes are half lines throughout (u8 ->
+        // u8 1080p radius 16 9.0 us, ordinary and tile by tile along the rows
+        // 10.4; 4096 x 4096 17 x 9 taps 15.2, 18.2).
         // Rows that do not start at 128-byte lines take ordinary stores where
         // strips meet in a line (store_rows) or, where no line lies within a
         // strip's row or in a one-round launch, throughout (one-round 1080 x
         // 1923 f32 16.6 us, split 20.9).
-        const int64_t pitch64 = int64_t(a.ostride[k]) * ST::ES;
-        const int pitch = int(pitch64);         // wraps only where a.far keeps it unused
-        const uintptr_t base = a.obase[k] + uintptr_t(y0 * pitch64 + int64_t(x0) * ST::ES);
-        const int rv = a.r[v], rh = a.r[h];
-        const int x = x0 + c0, xa = rh - x, xb = a.ncol - rh - x;          // valid pixels of the chunk: [xa, xb)
-        // An image hardly wider than its border may cut a chunk at both ends: the
-        // plain form below.  (A loop over such a chunk's pixels here cost the u8
-        // -> u8 launches 66 spilled vector registers: 3840 x 2160 radius 16 42
-        // us, 27 without it.)
-        const bool narrow = a.ncol - 2 * rh < ST::EPL;
-        if ((ST::ES == 4 || a.aligned) && !a.far && !narrow) {
-            const __amdgpu_buffer_rsrc_t orsrc =
-                __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base), short(0), 0x7fffffff, BUF_DWORD3);
+        constexpr bool LOOP = CPOL == CPOL_NT, ROWS = ST::ES == 4 && LOOP;
+        const auto rsrc_of = [](uintptr_t base) {
+            return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base), short(0), 0x7fffffff, BUF_DWORD3);
+        };
+        // the strip's chunks through a buffer at base, those where valid(i) holds
+        const auto chunks = [&](auto cp, uintptr_t base, int pitch, const auto& valid) {
+            constexpr int CP = cp;
+            const __amdgpu_buffer_rsrc_t orsrc = rsrc_of(base);
             const int off = r0 * pitch + c0 * ST::ES;
-            constexpr bool ROWS = ST::ES == 4 && CPOL == CPOL_NT;
-            // row steps of the mask rows, at lanes where in holds
-            const auto chunks = [&](auto cp, bool in, unsigned rows) {
-                constexpr int CP = cp;
+#pragma unroll
+            for (int i = 0; i < ST::NI; ++i)
+                __builtin_amdgcn_raw_buffer_store_b128(
+                    *reinterpret_cast<const v4u32_any*>(src + i * ST::RPI * ST::PITCH), orsrc,
+                    valid(i) ? off + i * ST::RPI * pitch : MINVALID, 0, CP);
+        };
+        const auto streaming = std::integral_constant<int, CPOL>{};
+        const auto ordinary = std::integral_constant<int, 0>{};
+        // any strip, with c the launch's arguments
+        const auto edge = [&](const auto& c) {
+            const int64_t pitch64 = int64_t(c.ostride[k]) * ST::ES;
+            const int pitch = int(pitch64);         // wraps only where c.far keeps it unused
+            const uintptr_t base = c.obase[k] + uintptr_t(y0 * pitch64 + int64_t(x0) * ST::ES);
+            const int rv = c.r[v], rh = c.r[h];
+            const bool buf = (ST::ES == 4 || c.aligned) && !c.far;
+            // the valid columns of the strip: [e0, e1)
+            const int e0 = max(rh - x0, 0), e1 = min(c.ncol - rh - x0, MSTRIP_W);
+            const bool cut = ((e0 | e1) & (ST::EPL - 1)) != 0;      // uniform: an edge lies within a chunk
+            const int yv = y0 + r0 - rv, rows = c.nrow - 2 * rv;    // row step i is valid: yv + RPI i in [0, rows)
+            // A chunk that an edge cuts is moved inside, where it overlaps its
+            // neighbour, with the same values.  (What a branch needs is computed
+            // in it: shared, it is held in scalar registers, 294 spilled in the
+            // f32 tile loop of radius class 8, 160 so.)
+            if constexpr (ST::ES == 4) {
+                if (buf && cut && e1 - e0 >= ST::EPL) {
+                    const int cs = min(max(c0, e0), e1 - ST::EPL);
+                    const bool in = c0 + ST::EPL > e0 && c0 < e1;
+                    const __amdgpu_buffer_rsrc_t orsrc = rsrc_of(base);
+                    const int off = r0 * pitch + cs * ST::ES;
+#pragma unroll
+                    for (int i = 0; i < ST::NI; ++i)
+                        __builtin_amdgcn_raw_buffer_store_b128(
+                            *reinterpret_cast<const v4u32u*>(src + i * ST::RPI * ST::PITCH + (cs - c0) * ST::ES), orsrc,
+                            in && unsigned(yv + i * ST::RPI) < unsigned(rows) ? off + i * ST::RPI * pitch : MINVALID, 0, 0);
+                    return;
+                }
+            }
+            if (buf && !cut) {
+                const auto valid = [&](int i) {
+                    return c0 >= e0 && c0 < e1 && unsigned(yv + i * ST::RPI) < unsigned(rows);
+                };
+                const int b0 = e0 * ST::ES, b1 = e1 * ST::ES;   // the strip's part of its lines
+                const bool whole = ST::ES < 4 ? true
+                                   : LOOP     ? ((b0 | b1) & 127) == 0
+                                              : (b0 & 63) == 0 && ((b1 & 63) == 0 || (RC == 16 && (b1 & 127) >= 112));
+                if (c.lines && whole) chunks(streaming, base, pitch, valid);
+                else                  chunks(ordinary, base, pitch, valid);
+            } else if (e1 - e0 >= ST::EPL) {
+                // an edge within a chunk of 16-bit or 8-bit pixels, rows of them
+                // that are not aligned to four, rows too far apart: plain addresses
+                const int cs = min(max(c0, e0), e1 - ST::EPL);
+                const bool in = c0 + ST::EPL > e0 && c0 < e1;
 #pragma unroll
                 for (int i = 0; i < ST::NI; ++i)
-                    __builtin_amdgcn_raw_buffer_store_b128(
-                        *reinterpret_cast<const v4u32_any*>(src + i * ST::RPI * ST::PITCH), orsrc,
-                        in && (rows >> i & 1u) ? off + i * ST::RPI * pitch : MINVALID, 0, CP);
-            };
-            const auto streaming = std::integral_constant<int, CPOL>{};
-            const auto ordinary = std::integral_constant<int, 0>{};
-            if (fast) {
-                if (a.lines)   chunks(streaming, true, ~0u);
-                else if (ROWS) store_rows<ST::PITCH>(orsrc, base, src, r0, c0 * ST::ES, pitch);
-                else           chunks(ordinary, true, ~0u);
+                    if (in && unsigned(yv + i * ST::RPI) < unsigned(rows))
+                        *reinterpret_cast<gptr<v4u32u>>(base + uintptr_t((i * ST::RPI + r0) * pitch64 + cs * ST::ES)) =
+                            *reinterpret_cast<const v4u32u*>(src + i * ST::RPI * ST::PITCH + (cs - c0) * ST::ES);
             } else {
-                const int lo = max(xa, 0), hi = min(xb, ST::EPL);
-                const bool in = lo == 0 && hi == ST::EPL;
-                unsigned rows = 0;                  // row steps inside the valid rows
+                // less than a chunk
 #pragma unroll
-                for (int i = 0; i < ST::NI; ++i) {
-                    const int y = y0 + i * ST::RPI + r0;
-                    rows |= unsigned(y >= rv && y < a.nrow - rv) << i;
-                }
-                const bool cut = !in && hi > lo;
-                const bool cuts = __builtin_amdgcn_ballot_w64(cut) != 0;
-                // the valid bytes of the strip's row: [e0, e1)
-                const int e0 = max(rh - x0, 0) * ST::ES, e1 = min(a.ncol - rh - x0, MSTRIP_W) * ST::ES;
-                constexpr int WHOLE = ST::ES < 4 ? 16 : CPOL == CPOL_NT ? 128 : 64;
-                if (a.lines && ((e0 | e1) & (WHOLE - 1)) == 0) chunks(streaming, in, rows);
-                else                                           chunks(ordinary, in, rows);
-                if (cuts)
-                    store_cut<ST::ES, 0, ST::NI>(orsrc, src, ST::RPI * ST::PITCH, off, ST::RPI * pitch, lo > 0,
-                                                 cut ? hi - lo : 0, rows);
+                for (int i = 0; i < ST::NI; ++i)
+                    if (unsigned(yv + i * ST::RPI) < unsigned(rows))
+                        store_chunk<ST::ES>(base + uintptr_t((i * ST::RPI + r0) * pitch64 + c0 * ST::ES),
+                                            src + i * ST::RPI * ST::PITCH, e0 - c0, e1 - c0);
+            }
+        };
+        if constexpr (LOOP) {
+            if (fast && (ST::ES == 4 || a.aligned) && !a.far) {
+                const int pitch = a.ostride[k] * ST::ES;
+                const uintptr_t base = a.obase[k] + uintptr_t(int64_t(y0) * pitch + int64_t(x0) * ST::ES);
+                const auto all = [](int) { return true; };
+                if (a.lines)             chunks(streaming, base, pitch, all);
+                else if constexpr (ROWS) store_rows<ST::PITCH>(rsrc_of(base), base, src, r0, c0 * ST::ES, pitch);
+                else                     chunks(ordinary, base, pitch, all);
+            } else if constexpr (sizeof(IN) < 4) {
+                edge(opaque_args(a));
+            } else {
+                edge(a);
             }
         } else {
-            // 16-bit and 8-bit rows that are not aligned to four pixels, rows
-            // too far apart, narrow images: plain addresses, ordinary stores
-#pragma unroll
-            for (int i = 0; i < ST::NI; ++i) {
-                const int row = i * ST::RPI + r0, y = y0 + row;
-                if (y < rv || y >= a.nrow - rv) continue;
-                store_chunk<ST::ES>(base + uintptr_t(row * pitch64 + c0 * ST::ES), src + i * ST::RPI * ST::PITCH, xa, xb);
-            }
+            edge(a);
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
         __builtin_amdgcn_wave_barrier();
