@@ -104,7 +104,7 @@ def hot_kernel_us(g, ins, outs, launches: int = LAUNCHES_PER_GRAPH, reps: int = 
     return e0.elapsed_time(e1) * 1000 / (reps * launches)
 
 
-# Sources that define the headline kernel (sepfir_mfma_kernel<16, 2, float,
+# Sources that define the headline kernel (sepfir_mfma_kernel<16, 4, float,
 # float, MODE_GAUSS>) and its launch: the recorded HBM traffic is reported
 # only while they hash as they did when the counters were taken.
 KERNEL_SOURCES = ("tucuda_amd/csrc/mfma.h", "tucuda_amd/csrc/sepfir.h", "tucuda_amd/csrc/batch.h",

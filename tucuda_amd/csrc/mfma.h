@@ -1453,11 +1453,11 @@ sepfir_mfma_loop_kernel(const SepArgs a, int ntiles)
     int t = mfma_share_lo(ntiles, grid, x) + b / QN;
     float* const stage = reinterpret_cast<float*>(stage4) + (threadIdx.x >> 6) * 16 * MOPITCH;
     if (t >= hi) return;                            // uniform over the workgroup
-    // The six-output strip code takes its lane index afresh in each tile: left to itself the compiler computes the lane-derived
-    // offsets once, before the loop, and holds them through it (3840 x 2160
-    // six outputs f32 1 % faster).  The one-output loop does so for 16-bit input
-    // at radius class 16 alone (4096 x 4096 bf16 29.4 against 31.4 us): u8 runs
-    // 3-7 % slower so.
+    // The six-output strip code takes its lane index afresh in each tile: left to
+    // itself the compiler computes the lane-derived offsets once, before the loop,
+    // and holds them through it (3840 x 2160 six outputs f32 1 % faster).  The
+    // one-output loop does so for 16-bit input at radius class 16 alone (4096 x
+    // 4096 bf16 29.4 against 31.4 us): u8 runs 3-7 % slower so.
     constexpr bool FRESH = MODE == MODE_GAUSS || (sizeof(IN) == 2 && RC == 16);
     // The next window goes into LDS before the tile's first stores, so that the
     // wait for its loads is not one for the stores too.
