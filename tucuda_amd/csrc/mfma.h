@@ -1153,9 +1153,11 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& 
         // 1192 f32 six outputs, radius 16: 15.0 us with the pieces of a cut chunk
         // stored one by one, 13.3 so; 823 x 519 11.4 -> 9.1, bf16 9.9 -> 8.0).
         // A tile loop takes the strips inside the valid region first, without
-        // these conditions, and for narrow input reads what the others need from
-        // the arguments there and then (held through the loop it spilled 38
-        // scalar registers: 3840 x 2160 u8 -> f32 42.4 us, 41.8 so).
+        // these conditions, and reads what the others need from the arguments
+        // there and then (held through the loop it spilled 38 scalar registers
+        // more: 3840 x 2160 u8 -> f32 42.4 us, 41.8 so; f32 52.6 against 51.7,
+        // 2560 x 1440 radius 12 29.4 against 28.4, 4096 x 4096 9 x 9 taps 35.8
+        // against 34.9).
         // Where the edge lies within a line, the strip writes a part of it:
         // streamed, that part goes to memory by itself, stored ordinarily it
         // stays in L2 until the kernel ends.  Float strips stream whole lines in
@@ -1257,10 +1259,8 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& 
                 if (a.lines)             chunks(streaming, base, pitch, all);
                 else if constexpr (ROWS) store_rows<ST::PITCH>(rsrc_of(base), base, src, r0, c0 * ST::ES, pitch);
                 else                     chunks(ordinary, base, pitch, all);
-            } else if constexpr (sizeof(IN) < 4) {
-                edge(opaque_args(a));
             } else {
-                edge(a);
+                edge(opaque_args(a));
             }
         } else {
             edge(a);
