@@ -1553,19 +1553,15 @@ int mfma_resident(K kernel)
 
 // Workgroups of a tile loop over n tiles, at most resident of them: the
 // fewest per CU that take no more rounds (2560 x 1440 u8 -> f32 six outputs,
-// radius 16: 22.5 us, 24.9 with all that fit).  TWO: of at most three rounds,
-// two workgroups per CU where they leave no more places idle -- six outputs
-// f32 -> f32, radius class 8, which the write stream bounds whether two or three
-// are resident, so that the emptier last round shows (3840 x 2160, 2040 tiles,
-// four rounds of 512 against three of 768: 44.7 -> 43.9 us; 3000 x 1500 27.6 ->
-// 26.7; with more rounds it goes either way: 4608 x 3456 86.8 -> 84.1, 4000 x
-// 4000 86.6 -> 89.9).
-template <bool TWO> int mfma_loop_grid(int n, int resident)
+// radius 16: 22.5 us, 24.9 with all that fit).  (Six outputs f32 -> f32,
+// radius class 8, with two per CU where the last of at most three rounds of three
+// is half empty: 3840 x 2160 51.9 us against 49.4 with three, 2000 x 4096 52.0
+// against 49.5, 3000 x 1500 30.3 against 29.0.)
+inline int mfma_loop_grid(int n, int resident)
 {
     static const int ncu = mfma_cus();
-    const auto rounds = [&](int64_t grid) { return (int64_t(n) + grid - 1) / grid; };
-    int64_t per_cu = (n + rounds(resident) * ncu - 1) / (rounds(resident) * ncu);
-    if (TWO && per_cu > 2 && rounds(per_cu * ncu) <= 3 && rounds(2 * ncu) * 2 <= rounds(per_cu * ncu) * per_cu) per_cu = 2;
+    const int64_t rounds = (int64_t(n) + resident - 1) / resident;
+    const int64_t per_cu = (n + rounds * ncu - 1) / (rounds * ncu);
     return int(std::min<int64_t>({int64_t(n), int64_t(resident), per_cu * ncu}));
 }
 
@@ -1588,14 +1584,13 @@ hipError_t launch_sepfir_mfma(const SepArgs& a, int nblocks, hipStream_t s)
                                      mfma_cus() * MFMA_LOOP_PER_CU<RC, IN, MODE>);
     static const int one = MODE == MODE_TAPS ? mfma_resident(sepfir_mfma_kernel<RC, WYR, IN, OUT, MODE>) : loop;
     constexpr int H = 16 * WYR, W = MSTRIP_W * (MWAVES / WYR);
-    constexpr bool TWO = MODE == MODE_GAUSS && RC == 8 && sizeof(IN) == 4 && sizeof(OUT) == 4;
     SepArgs r = a;
     r.tiles_y = (a.cy1 - a.cy0 + H - 1) / H;
     const int64_t n = int64_t((a.cx1 - a.cx0 + W - 1) / W) * r.tiles_y;
     if (n <= one)
         hipLaunchKernelGGL((sepfir_mfma_kernel<RC, WYR, IN, OUT, MODE>), dim3(int(n)), dim3(64 * MWAVES), 0, s, r);
     else
-        hipLaunchKernelGGL((sepfir_mfma_loop_kernel<RC, WYL, IN, OUT, MODE>), dim3(mfma_loop_grid<TWO>(nblocks, loop)),
+        hipLaunchKernelGGL((sepfir_mfma_loop_kernel<RC, WYL, IN, OUT, MODE>), dim3(mfma_loop_grid(nblocks, loop)),
                            dim3(64 * MWAVES), 0, s, a, nblocks);
     return hipGetLastError();
 }
