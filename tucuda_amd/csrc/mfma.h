@@ -1160,14 +1160,19 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& 
         // against 34.9).
         // Where the edge lies within a line, the strip writes a part of it:
         // streamed, that part goes to memory by itself, stored ordinarily it
-        // stays in L2 until the kernel ends.  Float strips stream whole lines in
-        // the tile loops, in a one-round launch also halves and, at radius class
-        // 16, lines that lack their last 16 bytes alone (six outputs f32,
-        // streaming against ordinary: 1080p radius 4, 16 bytes cut at the left,
-        // 14.4 against 12.6 us, and the last 16 at the right alone 13.2 against
-        // 12.3; radius 16, half a line, 14.1 against 14.8, 1292 x 1192 the last 16
-        // bytes 11.6 against 12.7; 3840 x 2160 radius 4 47.5 against 43.3, radius
-        // 16 50.0 against 49.0).  16-bit strips stream it wherever no chunk is cut
+        // stays in L2 until the kernel ends.  In the tile loops a float strip
+        // streams the chunks of its whole lines and stores those of a line that is
+        // cut ordinarily (six outputs f32, 3840 x 2160 radius 4: all streamed 47.2
+        // us, all ordinary 42.8, so 42.8; 4096 x 4096 91, 94, 83; 2560 x 1440, no
+        // buffer in a cache, 24.4, 26.4, 24.6; 64 mixed images 272, 278, 257),
+        // except that f32 -> f32 of radius class 16 streams halves too (3000 x 1500
+        // radius 16, no buffer in a cache, 29.0 us so, 32.2 ordinarily).  A
+        // one-round launch streams the strips whose lines are whole or cut in half
+        // and, at radius class 16, lack the last 16 bytes alone (1080p radius 4, 16
+        // bytes cut at the left, streaming against ordinary 14.4 against 12.6 us,
+        // the last 16 at the right alone 13.2 against 12.3; radius 16, half a line,
+        // 14.1 against 14.8, 1292 x 1192 the last 16 bytes 11.6 against 12.7; line by
+        // line as the loops VGA radius 4 7.9 against 7.4).  16-bit strips stream it wherever no chunk is cut
         // (1080p bf16 radius 16, a quarter line, 11.1 us, ordinary 11.9), and so
         // do 8-bit ones, whose rows of 64 bytes are half lines throughout (u8 ->
         // u8 1080p radius 16 9.0 us, ordinary and tile by tile along the rows
@@ -1204,6 +1209,12 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& 
             const int e0 = max(rh - x0, 0), e1 = min(c.ncol - rh - x0, MSTRIP_W);
             const bool cut = ((e0 | e1) & (ST::EPL - 1)) != 0;      // uniform: an edge lies within a chunk
             const int yv = y0 + r0 - rv, rows = c.nrow - 2 * rv;    // row step i is valid: yv + RPI i in [0, rows)
+            const int b0 = e0 * ST::ES, b1 = e1 * ST::ES;           // the strip's part of its lines
+            // the lane's chunk lies in a line that the strip writes whole
+            const auto in_whole = [&] {
+                const int cb = c0 * ST::ES;
+                return cb >= ((b0 + 127) & ~127) && cb + 16 <= (b1 & ~127);
+            };
             // A chunk that an edge cuts is moved inside, where it overlaps its
             // neighbour, with the same values.  (What a branch needs is computed
             // in it: shared, it is held in scalar registers, 294 spilled in the
@@ -1214,11 +1225,22 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& 
                     const bool in = c0 + ST::EPL > e0 && c0 < e1;
                     const __amdgpu_buffer_rsrc_t orsrc = rsrc_of(base);
                     const int off = r0 * pitch + cs * ST::ES;
+                    const auto moved = [&](auto cp, bool at) {
+                        constexpr int CP = cp;
 #pragma unroll
-                    for (int i = 0; i < ST::NI; ++i)
-                        __builtin_amdgcn_raw_buffer_store_b128(
-                            *reinterpret_cast<const v4u32u*>(src + i * ST::RPI * ST::PITCH + (cs - c0) * ST::ES), orsrc,
-                            in && unsigned(yv + i * ST::RPI) < unsigned(rows) ? off + i * ST::RPI * pitch : MINVALID, 0, 0);
+                        for (int i = 0; i < ST::NI; ++i)
+                            __builtin_amdgcn_raw_buffer_store_b128(
+                                *reinterpret_cast<const v4u32u*>(src + i * ST::RPI * ST::PITCH + (cs - c0) * ST::ES), orsrc,
+                                at && unsigned(yv + i * ST::RPI) < unsigned(rows) ? off + i * ST::RPI * pitch : MINVALID, 0,
+                                CP);
+                    };
+                    if (LOOP && c.lines) {
+                        const bool wl = in_whole();
+                        moved(streaming, in && wl);
+                        moved(ordinary, in && !wl);
+                    } else {
+                        moved(ordinary, in);
+                    }
                     return;
                 }
             }
@@ -1226,12 +1248,18 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& 
                 const auto valid = [&](int i) {
                     return c0 >= e0 && c0 < e1 && unsigned(yv + i * ST::RPI) < unsigned(rows);
                 };
-                const int b0 = e0 * ST::ES, b1 = e1 * ST::ES;   // the strip's part of its lines
-                const bool whole = ST::ES < 4 ? true
-                                   : LOOP     ? ((b0 | b1) & 127) == 0
-                                              : (b0 & 63) == 0 && ((b1 & 63) == 0 || (RC == 16 && (b1 & 127) >= 112));
-                if (c.lines && whole) chunks(streaming, base, pitch, valid);
-                else                  chunks(ordinary, base, pitch, valid);
+                const bool stream = ST::ES < 4 ? true
+                                    : LOOP     ? ((b0 | b1) & (RC == 16 && sizeof(IN) == 4 ? 63 : 127)) == 0
+                                               : (b0 & 63) == 0 && ((b1 & 63) == 0 || (RC == 16 && (b1 & 127) >= 112));
+                if (c.lines && stream) {
+                    chunks(streaming, base, pitch, valid);
+                } else if (ROWS && c.lines) {
+                    const bool wl = in_whole();
+                    chunks(streaming, base, pitch, [&](int i) { return wl && valid(i); });
+                    chunks(ordinary, base, pitch, [&](int i) { return !wl && valid(i); });
+                } else {
+                    chunks(ordinary, base, pitch, valid);
+                }
             } else if (e1 - e0 >= ST::EPL) {
                 // an edge within a chunk of 16-bit or 8-bit pixels, rows of them
                 // that are not aligned to four, rows too far apart: plain addresses
