@@ -271,20 +271,6 @@ template <class OUT> struct MStage {
 
 typedef v4u32 v4u32u __attribute__((aligned(1), may_alias));
 
-// Stores the elements [xa, xb) (of 16 / ES, ES bytes each) of the chunk at q in
-// LDS at p, one by one (strips that hold less than a chunk).
-template <int ES> __device__ __forceinline__ void store_chunk(uintptr_t p, const char* q, int xa, int xb)
-{
-    constexpr int E = 16 / ES;
-    using T = std::conditional_t<ES == 4, uint32_t, std::conditional_t<ES == 2, uint16_t, uint8_t>>;
-#pragma unroll 1
-    for (int e = max(xa, 0); e < min(xb, E); ++e) {
-        if constexpr (ES == 4)      reinterpret_cast<gptr<T>>(p)[e] = reinterpret_cast<const u32_any*>(q)[e];
-        else if constexpr (ES == 2) reinterpret_cast<gptr<T>>(p)[e] = reinterpret_cast<const u16_any*>(q)[e];
-        else                        reinterpret_cast<gptr<T>>(p)[e] = reinterpret_cast<const uint8_t*>(q)[e];
-    }
-}
-
 // Stores a strip of float rows that do not start at 128-byte lines, 4 rows an
 // instruction (16 lanes of 16 bytes each), rows pitch bytes apart in the output
 // from base, PITCH in LDS from src (the lane's first chunk, c bytes into row
@@ -1271,12 +1257,16 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& 
                         *reinterpret_cast<gptr<v4u32u>>(base + uintptr_t((i * ST::RPI + r0) * pitch64 + cs * ST::ES)) =
                             *reinterpret_cast<const v4u32u*>(src + i * ST::RPI * ST::PITCH + (cs - c0) * ST::ES);
             } else {
-                // less than a chunk
+                // less than a chunk: a lane a pixel (six outputs of radius 4, 1291 x
+                // 1192 bf16 9.1 us, 823 x 519 f32 7.9; with the pixels of a row stored
+                // one after the other 11.0 and 10.1)
+                using T = std::conditional_t<ST::ES == 4, u32_any, std::conditional_t<ST::ES == 2, u16_any, uint8_t>>;
+                const int x = e0 + lane % ST::EPL, q = lane / ST::EPL;
 #pragma unroll
-                for (int i = 0; i < ST::NI; ++i)
-                    if (unsigned(yv + i * ST::RPI) < unsigned(rows))
-                        store_chunk<ST::ES>(base + uintptr_t((i * ST::RPI + r0) * pitch64 + c0 * ST::ES),
-                                            src + i * ST::RPI * ST::PITCH, e0 - c0, e1 - c0);
+                for (int i = 0; i < 16; i += 64 / ST::EPL)
+                    if (x < e1 && unsigned(y0 + q + i - rv) < unsigned(rows))
+                        *reinterpret_cast<gptr<T>>(base + uintptr_t((q + i) * pitch64 + x * ST::ES)) =
+                            *reinterpret_cast<const T*>(sb + (q + i) * ST::PITCH + x * ST::ES);
             }
         };
         if constexpr (LOOP) {
