@@ -1204,7 +1204,8 @@ mfma_filter(const A& a, int y0, int x0, const MfmaOps& p, const ModeTabs<MODE>& 
             // A chunk that an edge cuts is moved inside, where it overlaps its
             // neighbour, with the same values.  (What a branch needs is computed
             // in it: shared, it is held in scalar registers, 294 spilled in the
-            // f32 tile loop of radius class 8, 160 so.)
+            // f32 tile loop of radius class 8, 160 so, 121 with the arguments read
+            // here.)
             if constexpr (ST::ES == 4) {
                 if (buf && cut && e1 - e0 >= ST::EPL) {
                     const int cs = min(max(c0, e0), e1 - ST::EPL);
